@@ -2,7 +2,9 @@
 //
 // Replaces the assignment kernels of DMatDVecMultExpr (blaze/math/expressions/
 // DMatDVecMultExpr.h:408-458 dispatch, :528-850 small kernel, :887-1114 large kernel).
-// HBM-bound: A is streamed exactly once with 16-byte loads; x is re-read from L2.
+// HBM-bound: A is streamed exactly once with 16-byte loads; x is re-read from L2.  The loads need
+// element alignment only, so odd row lengths stream like even ones (16384 x 12289 fp32: 138 us =
+// 5.8 TB/s, 369 us with 4-byte loads).
 //
 // A group of G lanes owns R consecutive rows.  Every lane walks the row with a stride of
 // G*VW elements (VW = 2 for 16-byte loads of double, 4 for float/int32), keeping one partial
@@ -17,7 +19,9 @@
 namespace bzg {
 namespace {
 
-typedef int i4v __attribute__((ext_vector_type(4)));
+// 16 bytes that need only element alignment: gfx950 takes a 16-byte global access at any 4-byte
+// address, and a wavefront's 1 KB then touches nine 128-byte lines instead of eight
+typedef int i4u __attribute__((ext_vector_type(4), aligned(4)));
 
 template <typename T>
 struct Arith {
@@ -34,7 +38,7 @@ struct Arith<int32_t> {  // wrap-around arithmetic, like the unsigned reinterpre
   }
 };
 
-template <typename T, int G, int R, bool VEC>
+template <typename T, int G, int R>
 __global__ __launch_bounds__(256) void gemv_kernel(int M, int N, int KC, T alpha, const T* __restrict__ A,
                                                    long lda, const T* __restrict__ x, T beta,
                                                    T* __restrict__ y, T* __restrict__ part) {
@@ -53,26 +57,23 @@ __global__ __launch_bounds__(256) void gemv_kernel(int M, int N, int KC, T alpha
 #pragma unroll
   for (int r = 0; r < R; ++r) acc[r] = T(0);
 
-  int cs = c0;  // first column of the scalar pass
-  if (VEC) {
-    const int vend = c1 / VW;  // c0 is a multiple of VW
-    for (int v = c0 / VW + lane_in_group; v < vend; v += G) {
-      T xv[VW];
-      *reinterpret_cast<i4v*>(xv) = *reinterpret_cast<const i4v*>(x + (long)v * VW);
+  const int vend = c1 / VW;  // c0 is a multiple of VW
+  for (int v = c0 / VW + lane_in_group; v < vend; v += G) {
+    T xv[VW];
+    *reinterpret_cast<i4u*>(xv) = *reinterpret_cast<const i4u*>(x + (long)v * VW);
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (row0 + r < M) {
-          T av[VW];
-          *reinterpret_cast<i4v*>(av) =
-              __builtin_nontemporal_load(reinterpret_cast<const i4v*>(A + (row0 + r) * lda + (long)v * VW));
+    for (int r = 0; r < R; ++r) {
+      if (row0 + r < M) {
+        T av[VW];
+        *reinterpret_cast<i4u*>(av) =
+            __builtin_nontemporal_load(reinterpret_cast<const i4u*>(A + (row0 + r) * lda + (long)v * VW));
 #pragma unroll
-          for (int e = 0; e < VW; ++e) acc[r] = AR::add(acc[r], AR::mul(av[e], xv[e]));
-        }
+        for (int e = 0; e < VW; ++e) acc[r] = AR::add(acc[r], AR::mul(av[e], xv[e]));
       }
     }
-    cs = vend * VW;  // tail columns (N not a multiple of VW)
   }
-  for (int c = cs + lane_in_group; c < c1; c += G) {
+  // tail columns (N not a multiple of VW)
+  for (int c = max(c0, vend * VW) + lane_in_group; c < c1; c += G) {
     const T xc = x[c];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -142,13 +143,13 @@ void launch_partials_reduce(bzg_context* ctx, int N, int P, T alpha, const T* pa
 }
 
 constexpr int kGemvTargetGroups = 2048;  // workgroups that keep every CU streaming
+constexpr int kGemvTTargetGroups = 4096;  // ... of the transposed form (4096: 152 us, 2048: 161 us, at 16384 x 12289 fp32)
 constexpr int kGemvMaxParts = 2048;      // partial sums per output entry
 
 template <typename T, int G, int R>
 bzg_status launch_gemv(bzg_context* ctx, int m, int n, T alpha, const T* A, long lda, const T* x,
                        T beta, T* y) {
   constexpr int VW = 16 / sizeof(T);
-  const bool vec = ((uintptr_t)A % 16 == 0) && ((uintptr_t)x % 16 == 0) && (lda % VW == 0);
   const long groups = (m + R - 1) / R;
   const long threads = groups * G;
   const long blocks = (threads + 255) / 256;
@@ -173,12 +174,8 @@ bzg_status launch_gemv(bzg_context* ctx, int m, int n, T alpha, const T* A, long
     part = static_cast<T*>(w);
   }
   const dim3 grid((unsigned)blocks, (unsigned)ks);
-  if (vec)
-    hipLaunchKernelGGL((gemv_kernel<T, G, R, true>), grid, dim3(256), 0, ctx->stream, m, n, kc, alpha, A, lda, x,
-                       beta, y, part);
-  else
-    hipLaunchKernelGGL((gemv_kernel<T, G, R, false>), grid, dim3(256), 0, ctx->stream, m, n, kc, alpha, A, lda, x,
-                       beta, y, part);
+  hipLaunchKernelGGL((gemv_kernel<T, G, R>), grid, dim3(256), 0, ctx->stream, m, n, kc, alpha, A, lda, x, beta, y,
+                     part);
   if (ks > 1) launch_partials_reduce<T>(ctx, m, ks, alpha, part, beta, y);
   BZG_LAUNCH_CHECK();
   return BZG_OK;
@@ -221,12 +218,16 @@ bzg_status gemv_dispatch(bzg_context* ctx, int64_t m, int64_t n, T alpha, const 
 // Transposed GEMV, y = alpha * A^T * x + beta * y for a row-major m x n A (y has n entries):
 // the column-major form of the product (TDMatDVecMultExpr).  Stage 1: a workgroup is CT
 // column threads by RL = 256 / CT row lanes; column thread c owns VW adjacent columns (one
-// 16-byte load per row when aligned), workgroup (cx, ry) covers columns
-// [cx CT VW, (cx + 1) CT VW) and, in row lane l, the rows (ry RL + l) + k RY RL.  x[i] is the
-// same for every column thread of a row lane.  Each thread keeps its column sums in row order;
-// the RL row lanes are added in lane order through LDS and written to part[ry][j].  Stage 2
-// adds the RY partials of column j in index order, so the result is identical run to run.
-template <typename T, bool VEC>
+// 16-byte load per row, whatever the row's alignment), workgroup (cx, ry) covers columns
+// [cx CT VW, (cx + 1) CT VW) and, in row lane l, the rows ry CH + l + k RL of its chunk of CH
+// consecutive rows.  Bound by memory: 16384 x 12289 fp32 (rows of odd length, so no row but the
+// first is 16-byte aligned) runs in 149 us = 5.4 TB/s; with four 4-byte loads for such rows it was
+// 258 us, with rows dealt out round-robin instead of in chunks 155 us (aligned rows: 139 against
+// 154).  x[i] is the same for every column thread of a row lane.  Each thread keeps its column
+// sums in row order; the RL row lanes are added in lane order through LDS and written to
+// part[ry][j].  Stage 2 adds the RY partials of column j in index order, so the result is
+// identical run to run.
+template <typename T>
 __global__ __launch_bounds__(256) void gemv_t_partial_kernel(int M, int N, const T* __restrict__ A, long lda,
                                                              const T* __restrict__ x, T* __restrict__ part,
                                                              int ct_log2) {
@@ -236,24 +237,25 @@ __global__ __launch_bounds__(256) void gemv_t_partial_kernel(int M, int N, const
   const int CT = 1 << ct_log2, RL = 256 >> ct_log2;
   const int ct = threadIdx.x & (CT - 1), rl = threadIdx.x >> ct_log2;
   const long j = ((long)blockIdx.x * CT + ct) * VW;
-  const long step = (long)gridDim.y * RL;
+  const long ch = ((M + gridDim.y - 1) / gridDim.y + RL - 1) / RL * RL;
+  const long i0 = (long)blockIdx.y * ch, i1 = min((long)M, i0 + ch);
   T s[VW];
 #pragma unroll
   for (int e = 0; e < VW; ++e) s[e] = T(0);
   if (j < N) {
-    if (VEC && j + VW <= N) {
+    if (j + VW <= N) {
 #pragma unroll 8
-      for (long i = (long)blockIdx.y * RL + rl; i < M; i += step) {
+      for (long i = i0 + rl; i < i1; i += RL) {
         const T xi = x[i];
         T av[VW];
-        *reinterpret_cast<i4v*>(av) = __builtin_nontemporal_load(reinterpret_cast<const i4v*>(A + i * lda + j));
+        *reinterpret_cast<i4u*>(av) = __builtin_nontemporal_load(reinterpret_cast<const i4u*>(A + i * lda + j));
 #pragma unroll
         for (int e = 0; e < VW; ++e) s[e] = AR::add(s[e], AR::mul(av[e], xi));
       }
     } else {
       const int w = (int)min((long)VW, N - j);
 #pragma unroll 4
-      for (long i = (long)blockIdx.y * RL + rl; i < M; i += step) {
+      for (long i = i0 + rl; i < i1; i += RL) {
         const T xi = x[i];
         const T* row = A + i * lda + j;
 #pragma unroll
@@ -296,7 +298,6 @@ bzg_status gemv_t_dispatch(bzg_context* ctx, int64_t m, int64_t n, T alpha, cons
   }
   BZG_REQUIRE(A != nullptr && x != nullptr, BZG_ERR_INVALID_ARGUMENT, "gemv: null A or x");
   constexpr int VW = 16 / sizeof(T);
-  const bool vec = ((uintptr_t)A % 16 == 0) && (lda % VW == 0);
   // column threads: the next power of two covering the row, at most 256 (the workgroup)
   int ct_log2 = 0;
   while (ct_log2 < 8 && ((int64_t)VW << ct_log2) < n) ++ct_log2;
@@ -304,19 +305,15 @@ bzg_status gemv_t_dispatch(bzg_context* ctx, int64_t m, int64_t n, T alpha, cons
   const int64_t cx = (n + ct * VW - 1) / (ct * VW);
   // row partitions: enough workgroups to fill the chip, at least 16 rows per row lane
   const int64_t ry = std::max<int64_t>(1, std::min<int64_t>({(int64_t)kGemvMaxParts, (m + 16 * rl - 1) / (16 * rl),
-                                                            (kGemvTargetGroups + cx - 1) / cx}));
+                                                            (kGemvTTargetGroups + cx - 1) / cx}));
   BZG_REQUIRE(cx < (1LL << 31), BZG_ERR_UNSUPPORTED, "gemv: too many columns");
   void* w = nullptr;
   bzg_status st = workspace(ctx, 11, (size_t)ry * n * sizeof(T), &w);
   if (st) return st;
   T* part = static_cast<T*>(w);
   const dim3 grid((unsigned)cx, (unsigned)ry);
-  if (vec)
-    hipLaunchKernelGGL((gemv_t_partial_kernel<T, true>), grid, dim3(256), 0, ctx->stream, (int)m, (int)n, A,
-                       (long)lda, x, part, ct_log2);
-  else
-    hipLaunchKernelGGL((gemv_t_partial_kernel<T, false>), grid, dim3(256), 0, ctx->stream, (int)m, (int)n, A,
-                       (long)lda, x, part, ct_log2);
+  hipLaunchKernelGGL((gemv_t_partial_kernel<T>), grid, dim3(256), 0, ctx->stream, (int)m, (int)n, A, (long)lda, x,
+                     part, ct_log2);
   launch_partials_reduce<T>(ctx, (int)n, (int)ry, alpha, part, beta, y);
   BZG_LAUNCH_CHECK();
   return BZG_OK;
