@@ -419,7 +419,7 @@ bzg_status bzg_batched_order(bzg_context* ctx, int64_t count, const int32_t* n_h
  * ipiv (n entries) and info (one entry) DEVICE arrays.  P A = L U as LAPACK dgetrf computes it
  * for A: ipiv 1-based in interchange order, info = 0 or the 1-based column of the first exactly
  * zero pivot (the factorisation completes).  The products inside run on bzg_dgemm; workspace
- * (n ints + n * nrhs doubles for the solves) is cached in the context.  Orders above 32768 return
+ * (20 bytes per row + n * nrhs doubles for the solves, twice that for nrhs <= 64) is cached in the context.  Orders above 32768 return
  * BZG_ERR_UNSUPPORTED. */
 /* dgetrf: A := L \ U in place (replaces getrf, blaze/math/lapack/clapack/getrf.h:190-197 and
  * the factorisation under lu(), blaze/math/dense/LU.h:98-140). */
@@ -428,8 +428,8 @@ bzg_status bzg_dgetrf(bzg_context* ctx, int64_t n, double* A, int64_t lda, int32
 bzg_status bzg_dgetrs(bzg_context* ctx, int64_t n, int64_t nrhs, const double* A, int64_t lda,
                       const int32_t* ipiv, double* B, int64_t ldb);
 /* dgesv = dgetrf + dgetrs (replaces solve() for one system: blaze/math/dense/LSE.h:6343-6373 ->
- * solveNxN LSE.h:5229-5257 -> dgesv_, clapack/gesv.h:207).  B is left unchanged when info > 0;
- * reading info back synchronises the context stream once. */
+ * solveNxN LSE.h:5229-5257 -> dgesv_, clapack/gesv.h:207).  B is left unchanged when info > 0
+ * (decided on the device: the call does not synchronise). */
 bzg_status bzg_dgesv(bzg_context* ctx, int64_t n, int64_t nrhs, double* A, int64_t lda, int32_t* ipiv,
                      double* B, int64_t ldb, int32_t* info);
 /* A := A^-1 from bzg_dgetrf's factors (info must have been 0): the inverse by LU of invert()
