@@ -6,8 +6,12 @@
 // FP64 / FP32: MFMA 16x16x4 tiles (v_mfma_f64_16x16x4f64, v_mfma_f32_16x16x4f32).  A workgroup
 // of 4 wavefronts computes a BM x BN tile of C; each wave owns a WM x WN sub-tile held in
 // MFMA accumulators.  A and B K-slabs of depth BK are staged through LDS with two buffers:
-// global loads of slab t+1 are issued into registers before the MFMAs of slab t and written
-// to the idle LDS buffer afterwards, so one barrier per slab suffices.
+// global loads of the next slab (small tiles: the next two) are in flight in registers during the
+// MFMAs of a slab and written to the idle LDS buffer afterwards, so one barrier per slab suffices.
+// Small tiles are bound by that latency, so their slabs are deep (256 bytes of k for 32 x 32, 128 for
+// 64 x 64): 512^3 FP64 9.7 us = 27.7 TFLOP/s (22.7 us with 16 of k, one slab ahead), 1024^3 FP32
+// 27 us (39.8), 1523 x 1777 x 2021 FP32 with odd leading dimensions 100 us (181: 4-byte loads).
+// Large tiles are bound by the matrix cores: 4096^3 68.2 TFLOP/s FP64, 134 FP32.
 // Every C element is produced by one wave in a fixed k order (no split-K, no atomics), so the
 // result is identical run to run and independent of the launch shape chosen for other calls.
 //
@@ -19,14 +23,12 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 
 namespace bzg {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kBK = 16;
-constexpr int kPadA = 1;   // A slab stored [BM][BK+1]: conflict-free fragment reads
-constexpr int kPadB = 16;  // B slab stored [BK][BN+16]
 
 template <typename T>
 struct Mfma;
@@ -51,15 +53,18 @@ struct Mfma<float> {
   __device__ static int row(int i, int lane) { return 4 * (lane / 16) + i; }
 };
 
+// 16 bytes of elements, element-aligned: gfx950 takes a 16-byte global access at any element address
 template <typename T>
-struct Vec2;
+struct Vec16;
 template <>
-struct Vec2<double> {
-  using type = double2;
+struct Vec16<double> {
+  typedef double type __attribute__((ext_vector_type(2), aligned(8)));
+  typedef double aligned_type __attribute__((ext_vector_type(2)));
 };
 template <>
-struct Vec2<float> {
-  using type = float2;
+struct Vec16<float> {
+  typedef float type __attribute__((ext_vector_type(4), aligned(4)));
+  typedef float aligned_type __attribute__((ext_vector_type(4)));
 };
 
 // Maps the linear workgroup id to a (tile_m, tile_n) pair.  Consecutive workgroup ids are
@@ -80,43 +85,55 @@ __device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, i
   tn = in_group / gsize;
 }
 
-template <typename T, int BM, int BN>
+// A slab stored [BM][BK + pad], B slab [BK][BN + pad].  Strides for which the fragment reads hit
+// distinct banks (A: 4 banks modulo 64 from row to row; B: rows k and k + 1 half the banks apart) and
+// rows start 16-byte aligned for vector stores.  A transposed operand is stored element by
+// element along the other direction: there the strides are 1 modulo 16 elements, so that the
+// rows a wavefront writes at once spread over 16 banks instead of 8 (A) or 1 (B).
+template <typename T, int BM, int BN, int BK, bool TA = false, bool TB = false>
 struct GemmShm {
-  T As[2][BM * (kBK + kPadA)];
-  T Bs[2][kBK * (BN + kPadB)];
+  static constexpr int LDA = TA ? (BK + 16) / 32 * 32 + 17 - (BK % 32 ? 32 : 0) : BK + 16 / (int)sizeof(T);
+  static constexpr int LDB = BN + (TB ? 17 : 16);
+  __align__(16) T As[2][BM * LDA];
+  __align__(16) T Bs[2][BK * LDB];
 };
 
 // One BM x BN tile (tm, tn) of C = alpha A B + beta C by the 4 wavefronts of the workgroup.
-// Every element of C is summed in the same k order (slabs of kBK, MFMA k-steps of 4) whatever
-// the tile shape, so all tile shapes give bit-identical results.
+// Every element of C is summed in the same k order (MFMA k-steps of 4) whatever the tile shape
+// and slab depth, so all tile shapes give bit-identical results.
 // TA / TB: A (B) is given transposed, i.e. stored k x m (n x k) row-major with leading
 // dimension lda >= m (ldb >= k); the slabs are then read along m (k) and transposed on the
 // way into LDS, so the MFMA loop and its summation order are the same for all four forms.
-template <typename T, int BM, int BN, int WM, int WN, bool VEC, bool TA = false, bool TB = false>
+//
+// PF slabs of global loads are in flight in registers ahead of the slab being multiplied.
+// The loads are 16 bytes at element alignment (odd leading dimensions take the same path).  Rows
+// past the matrix are read as its last row and columns past it as its last column: they feed
+// only elements of C that are not stored.  Only the last slab, if K is not a multiple of BK,
+// checks k (and is zero beyond K in both operands).
+template <typename T, int BM, int BN, int WM, int WN, int BK, int PF, bool TA = false, bool TB = false>
 __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T* __restrict__ A,
                                           long lda, const T* __restrict__ B, long ldb, T beta,
                                           T* __restrict__ C, long ldc, int tm, int tn,
-                                          GemmShm<T, BM, BN>& sh) {
+                                          GemmShm<T, BM, BN, BK, TA, TB>& sh) {
   using MF = Mfma<T>;
   using acc_t = typename MF::acc_t;
-  using V2 = typename Vec2<T>::type;
+  using VU = typename Vec16<T>::type;          // 16 bytes, element-aligned (global memory)
+  using VA = typename Vec16<T>::aligned_type;  // 16-byte aligned (LDS)
+  constexpr int VW = 16 / (int)sizeof(T);
   constexpr int WAVES_N = BN / WN;
   constexpr int FM = WM / 16;  // MFMA blocks per wave along m
   constexpr int FN = WN / 16;  // MFMA blocks per wave along n
-  constexpr int LDA_S = kBK + kPadA;
-  constexpr int LDB_S = BN + kPadB;
-  constexpr int NA = BM * kBK / (2 * kThreads);  // 2-element vectors per thread, A slab
-  constexpr int NB = kBK * BN / (2 * kThreads);  // 2-element vectors per thread, B slab
-  constexpr int A_VPR = kBK / 2;                 // vectors per A slab row
-  constexpr int A_RPP = kThreads / A_VPR;        // A rows per pass
-  constexpr int B_VPR = BN / 2;
-  constexpr int B_RPP = kThreads / B_VPR;
-  constexpr int AT_VPR = BM / 2;                 // transposed A: vectors per stored k row
-  constexpr int AT_RPP = kThreads / AT_VPR;
-  constexpr int BT_VPR = kBK / 2;                // transposed B: vectors per stored n row
-  constexpr int BT_RPP = kThreads / BT_VPR;
+  constexpr int LDA_S = GemmShm<T, BM, BN, BK, TA, TB>::LDA;
+  constexpr int LDB_S = GemmShm<T, BM, BN, BK, TA, TB>::LDB;
+  constexpr int NA = BM * BK / (VW * kThreads);  // vectors per thread, A slab
+  constexpr int NB = BK * BN / (VW * kThreads);  // vectors per thread, B slab
+  // stored rows of a slab: A [m][k] (TA: [k][m]), B [k][n] (TB: [n][k]); vectors per stored row and
+  // stored rows per pass of the workgroup
+  constexpr int A_VPR = (TA ? BM : BK) / VW, A_RPP = kThreads / A_VPR;
+  constexpr int B_VPR = (TB ? BK : BN) / VW, B_RPP = kThreads / B_VPR;
   static_assert(NA >= 1 && NB >= 1, "tile too small for 256 threads");
   static_assert((BM / WM) * (BN / WN) == 4, "four wavefronts per workgroup");
+  static_assert(PF == 1 || PF == 2, "one or two slabs ahead");
 
   auto& As = sh.As;
   auto& Bs = sh.Bs;
@@ -136,96 +153,97 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = acc_t{};
 
-  V2 ra[NA], rb[NB];
+  struct Regs {
+    VU a[NA], b[NB];
+  };
 
-  // thread-local (row, column) of vector i in the stored slab
-  auto a_rc = [&](int i, int& r, int& c) {
-    if (TA) { r = tid / AT_VPR + i * AT_RPP; c = (tid % AT_VPR) * 2; }  // r: k, c: m
-    else    { r = tid / A_VPR + i * A_RPP;   c = (tid % A_VPR) * 2; }   // r: m, c: k
-  };
-  auto b_rc = [&](int i, int& r, int& c) {
-    if (TB) { r = tid / BT_VPR + i * BT_RPP; c = (tid % BT_VPR) * 2; }  // r: n, c: k
-    else    { r = tid / B_VPR + i * B_RPP;   c = (tid % B_VPR) * 2; }   // r: k, c: n
-  };
-  auto load_slab = [&](int k0) {
-    const bool full = (m0 + BM <= M) && (n0 + BN <= N) && (k0 + kBK <= K);
-    if (VEC && full) {
-#pragma unroll
-      for (int i = 0; i < NA; ++i) {
-        int r, c;
-        a_rc(i, r, c);
-        ra[i] = TA ? *reinterpret_cast<const V2*>(A + (long)(k0 + r) * lda + m0 + c)
-                   : *reinterpret_cast<const V2*>(A + (long)(m0 + r) * lda + k0 + c);
-      }
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        int r, c;
-        b_rc(i, r, c);
-        rb[i] = TB ? *reinterpret_cast<const V2*>(B + (long)(n0 + r) * ldb + k0 + c)
-                   : *reinterpret_cast<const V2*>(B + (long)(k0 + r) * ldb + n0 + c);
-      }
+  // One slab of both operands.  A stored row or column outside its matrix is read as the last one
+  // (an address, never a selection: a selection would wait for the load); what lies beyond K is
+  // zeroed on the way into LDS.
+  const bool vec_a = !TA || m0 + BM <= M, vec_b = TB || n0 + BN <= N;
+  auto load_op = [&](auto rows_k, bool vec, const T* __restrict__ X, long ldx, int o0, int lim, int k0, int r0, int c0,
+                     VU& v) __attribute__((always_inline)) {
+    constexpr bool ROWS_K = decltype(rows_k)::value;  // stored rows run along k
+    if (vec) {
+      const long row = ROWS_K ? r0 : min(o0 + r0, lim - 1);
+      const T* p = X + row * ldx + (ROWS_K ? o0 + c0 : c0);
+      v = *reinterpret_cast<const VU*>(p + (ROWS_K ? (long)k0 * ldx : (long)k0));
     } else {
+      const int row = min((ROWS_K ? k0 : o0) + r0, (ROWS_K ? K : lim) - 1);
+      const int col = (ROWS_K ? o0 : k0) + c0, cmax = (ROWS_K ? lim : K) - 1;
+      const T* p = X + (long)row * ldx;
 #pragma unroll
-      for (int i = 0; i < NA; ++i) {
-        int r, c;
-        a_rc(i, r, c);
-        // stored row gr, stored columns gc, gc + 1 and their bounds
-        const int gr = TA ? k0 + r : m0 + r, gc = TA ? m0 + c : k0 + c;
-        const bool rin = gr < (TA ? K : M);
-        const int cl = TA ? M : K;
-        ra[i].x = (rin && gc < cl) ? A[(long)gr * lda + gc] : T(0);
-        ra[i].y = (rin && gc + 1 < cl) ? A[(long)gr * lda + gc + 1] : T(0);
-      }
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        int r, c;
-        b_rc(i, r, c);
-        const int gr = TB ? n0 + r : k0 + r, gc = TB ? k0 + c : n0 + c;
-        const bool rin = gr < (TB ? N : K);
-        const int cl = TB ? K : N;
-        rb[i].x = (rin && gc < cl) ? B[(long)gr * ldb + gc] : T(0);
-        rb[i].y = (rin && gc + 1 < cl) ? B[(long)gr * ldb + gc + 1] : T(0);
-      }
+      for (int e = 0; e < VW; ++e) v[e] = p[min(col + e, cmax)];
     }
   };
-  auto store_slab = [&](int buf) {
+  // `fast`: the slab is full and both operands are read by vectors, known at compile time
+  auto load_slab = [&](auto fast, int k0, Regs& r) __attribute__((always_inline)) {
+    constexpr bool FAST = decltype(fast)::value;
+    const bool kfull = k0 + BK <= K;
+    const bool va = FAST || (vec_a && kfull), vb = FAST || (vec_b && kfull);  // uniform
+    if (va) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+        load_op(std::integral_constant<bool, TA>{}, true, A, lda, m0, M, k0, tid / A_VPR + i * A_RPP, (tid % A_VPR) * VW,
+                r.a[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+        load_op(std::integral_constant<bool, TA>{}, false, A, lda, m0, M, k0, tid / A_VPR + i * A_RPP,
+                (tid % A_VPR) * VW, r.a[i]);
+    }
+    if (vb) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+        load_op(std::integral_constant<bool, !TB>{}, true, B, ldb, n0, N, k0, tid / B_VPR + i * B_RPP,
+                (tid % B_VPR) * VW, r.b[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+        load_op(std::integral_constant<bool, !TB>{}, false, B, ldb, n0, N, k0, tid / B_VPR + i * B_RPP,
+                (tid % B_VPR) * VW, r.b[i]);
+    }
+  };
+  auto store_slab = [&](auto fast, int buf, int k0, Regs& q) __attribute__((always_inline)) {
+    constexpr bool FAST = decltype(fast)::value;
+    if (!FAST && k0 + BK > K) {  // the last, partial slab
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int e = 0; e < VW; ++e)
+          if (k0 + (TA ? tid / A_VPR + i * A_RPP : (tid % A_VPR) * VW + e) >= K) q.a[i][e] = T(0);
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int e = 0; e < VW; ++e)
+          if (k0 + (TB ? (tid % B_VPR) * VW + e : tid / B_VPR + i * B_RPP) >= K) q.b[i][e] = T(0);
+    }
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      int r, c;
-      a_rc(i, r, c);
-      if (TA) {  // (k = r, m = c, c + 1) -> As[m][k]
-        As[buf][c * LDA_S + r] = ra[i].x;
-        As[buf][(c + 1) * LDA_S + r] = ra[i].y;
+      const int r = tid / A_VPR + i * A_RPP, c = (tid % A_VPR) * VW;
+      if (TA) {  // (k = r, m = c ..) -> As[m][k]
+#pragma unroll
+        for (int e = 0; e < VW; ++e) As[buf][(c + e) * LDA_S + r] = q.a[i][e];
       } else {
-        As[buf][r * LDA_S + c] = ra[i].x;
-        As[buf][r * LDA_S + c + 1] = ra[i].y;
+        *reinterpret_cast<VA*>(&As[buf][r * LDA_S + c]) = q.a[i];
       }
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      int r, c;
-      b_rc(i, r, c);
-      if (TB) {  // (n = r, k = c, c + 1) -> Bs[k][n]
-        Bs[buf][c * LDB_S + r] = rb[i].x;
-        Bs[buf][(c + 1) * LDB_S + r] = rb[i].y;
+      const int r = tid / B_VPR + i * B_RPP, c = (tid % B_VPR) * VW;
+      if (TB) {  // (n = r, k = c ..) -> Bs[k][n]
+#pragma unroll
+        for (int e = 0; e < VW; ++e) Bs[buf][(c + e) * LDB_S + r] = q.b[i][e];
       } else {
-        *reinterpret_cast<V2*>(&Bs[buf][r * LDB_S + c]) = rb[i];
+        *reinterpret_cast<VA*>(&Bs[buf][r * LDB_S + c]) = q.b[i];
       }
     }
   };
-
-  const int nk = (K + kBK - 1) / kBK;
-  load_slab(0);
-  store_slab(0);
-  __syncthreads();
-
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk) load_slab((kt + 1) * kBK);
+  auto multiply = [&](int buf) __attribute__((always_inline)) {
     const T* as = As[buf];
     const T* bs = Bs[buf];
 #pragma unroll
-    for (int kk = 0; kk < kBK; kk += 4) {
+    for (int kk = 0; kk < BK; kk += 4) {
       T a[FM], b[FN];
 #pragma unroll
       for (int i = 0; i < FM; ++i) a[i] = as[(wm0 + i * 16 + lane % 16) * LDA_S + kk + lane / 16];
@@ -236,8 +254,55 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = MF::mma(a[i], b[j], acc[i][j]);
     }
-    if (kt + 1 < nk) store_slab(buf ^ 1);
-    __syncthreads();
+  };
+
+  constexpr std::true_type fast{};
+  constexpr std::false_type any{};
+  const int nk = (K + BK - 1) / BK;
+  const int nfast = vec_a && vec_b ? K / BK : 0;  // full slabs, if read by vectors
+  Regs ra, rb;
+  load_slab(any, 0, ra);
+  if (PF == 2 && nk > 1) load_slab(any, BK, rb);
+  store_slab(any, 0, 0, ra);
+  __syncthreads();
+  int kt = 0;
+  if (PF == 1) {
+    // Past the end slab 0 is requested again: with the last load left out by a branch 4096^3 FP64
+    // takes 2.14 ms instead of 2.02 (and 2.11 as one basic block, where the compiler moves the loads
+    // down between the products).
+    for (; kt < nk; ++kt) {
+      load_slab(any, kt + 1 < nk ? (kt + 1) * BK : 0, ra);
+      multiply(kt & 1);
+      if (kt + 1 < nk) store_slab(any, (kt & 1) ^ 1, (kt + 1) * BK, ra);
+      __syncthreads();
+    }
+  } else {
+    // slab kt in LDS buffer kt & 1, slab kt + 1 on its way in the other register set, slab kt + 2
+    // requested into the set that held kt.  Full slabs in a loop without branches (2048^3 FP64, both
+    // operands transposed: 262 us, 302 with them; 512^3 9.7, 11.7).
+    for (; kt + 3 < nfast; kt += 2) {
+      load_slab(fast, (kt + 2) * BK, ra);
+      multiply(0);
+      store_slab(fast, 1, (kt + 1) * BK, rb);
+      __syncthreads();
+      load_slab(fast, (kt + 3) * BK, rb);
+      multiply(1);
+      store_slab(fast, 0, (kt + 2) * BK, ra);
+      __syncthreads();
+    }
+    // Past the end slab 0 is requested again: with a conditional load the wait for slab kt + 1 could
+    // not leave slab kt + 2 in flight.
+    for (; kt < nk; kt += 2) {
+      load_slab(any, kt + 2 < nk ? (kt + 2) * BK : 0, ra);
+      multiply(0);
+      if (kt + 1 < nk) store_slab(any, 1, (kt + 1) * BK, rb);
+      __syncthreads();
+      if (kt + 1 >= nk) break;
+      load_slab(any, kt + 3 < nk ? (kt + 3) * BK : 0, rb);
+      multiply(1);
+      if (kt + 2 < nk) store_slab(any, 0, (kt + 2) * BK, ra);
+      __syncthreads();
+    }
   }
 
   // Epilogue: C = alpha*acc + beta*C; beta == 0 never reads C (it may hold NaN/garbage).
@@ -259,22 +324,23 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
       }
 }
 
-template <typename T, int BM, int BN, int WM, int WN, bool VEC, bool TA = false, bool TB = false>
+template <typename T, int BM, int BN, int WM, int WN, int BK, int PF, bool TA = false, bool TB = false>
 __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(int M, int N, int K, T alpha,
                                                              const T* __restrict__ A, long lda,
                                                              const T* __restrict__ B, long ldb,
                                                              T beta, T* __restrict__ C,
                                                              long ldc) {
-  __shared__ GemmShm<T, BM, BN> sh;
+  __shared__ GemmShm<T, BM, BN, BK, TA, TB> sh;
   const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = (N + BN - 1) / BN;
   int tm, tn;
   tile_coords(tiles_m, tiles_n, tm, tn);
-  gemm_tile<T, BM, BN, WM, WN, VEC, TA, TB>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, sh);
+  gemm_tile<T, BM, BN, WM, WN, BK, PF, TA, TB>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, sh);
 }
 
 // ---- grouped GEMM: many independent products of uneven sizes in one persistent launch ----
 constexpr int kGT = 64;  // tile of the grouped kernel (64 x 64, waves of 32 x 32)
+constexpr int kGBK = 16;
 
 // Tiles of one problem; a problem that fails the bzg_dgemm argument rules gets none (and
 // status -1 when a status array is given), an empty one none (status 0).
@@ -322,7 +388,7 @@ __global__ __launch_bounds__(1024) void grouped_prefix_kernel(int count, const b
 // Problems with k == 0 are scaled (C = beta C) tile by tile.
 __global__ __launch_bounds__(kThreads, 2) void gemm_grouped_kernel(int count, const bzg_dgemm_problem* __restrict__ pr,
                                                                    const int64_t* __restrict__ prefix) {
-  __shared__ GemmShm<double, kGT, kGT> sh;
+  __shared__ GemmShm<double, kGT, kGT, kGBK> sh;
   const int64_t total = prefix[count];
   for (int64_t t = blockIdx.x; t < total; t += gridDim.x) {
     int lo = 0, hi = count - 1;  // last p with prefix[p] <= t
@@ -334,8 +400,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_grouped_kernel(int count, co
     const int tiles_n = (int)((q.n + kGT - 1) / kGT);
     const int local = (int)(t - prefix[lo]);
     const int tm = local / tiles_n, tn = local % tiles_n;
-    const bool vec = ((uintptr_t)q.A % 16 == 0) && ((uintptr_t)q.B % 16 == 0) && (q.lda % 2 == 0) &&
-                     (q.ldb % 2 == 0);
     if (q.k == 0) {
       for (int e = threadIdx.x; e < kGT * kGT; e += kThreads) {
         const long r = (long)tm * kGT + e / kGT, c = (long)tn * kGT + e % kGT;
@@ -344,12 +408,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_grouped_kernel(int count, co
           *p = (q.beta == 0.0) ? 0.0 : q.beta * *p;
         }
       }
-    } else if (vec) {
-      gemm_tile<double, kGT, kGT, 32, 32, true>((int)q.m, (int)q.n, (int)q.k, q.alpha, q.A, q.lda, q.B, q.ldb,
-                                                q.beta, q.C, q.ldc, tm, tn, sh);
     } else {
-      gemm_tile<double, kGT, kGT, 32, 32, false>((int)q.m, (int)q.n, (int)q.k, q.alpha, q.A, q.lda, q.B, q.ldb,
-                                                 q.beta, q.C, q.ldc, tm, tn, sh);
+      gemm_tile<double, kGT, kGT, 32, 32, kGBK, 2>((int)q.m, (int)q.n, (int)q.k, q.alpha, q.A, q.lda, q.B, q.ldb,
+                                                   q.beta, q.C, q.ldc, tm, tn, sh);
     }
     __syncthreads();  // LDS of this tile is free before the next one is staged
   }
@@ -440,21 +501,15 @@ bzg_status check_gemm_args(bzg_context* ctx, int64_t m, int64_t n, int64_t k, co
   return BZG_OK;
 }
 
-template <typename T, int BM, int BN, int WM, int WN, bool TA = false, bool TB = false>
+template <typename T, int BM, int BN, int WM, int WN, int BK, int PF, bool TA = false, bool TB = false>
 bzg_status launch_tile(bzg_context* ctx, int m, int n, int k, T alpha, const T* A, long lda,
                        const T* B, long ldb, T beta, T* C, long ldc) {
-  const bool vec = ((uintptr_t)A % (2 * sizeof(T)) == 0) && ((uintptr_t)B % (2 * sizeof(T)) == 0) &&
-                   (lda % 2 == 0) && (ldb % 2 == 0);
   ProfScope prof(ctx, sizeof(T) == 8 ? "dgemm" : "sgemm");
   const long tiles = (long)((m + BM - 1) / BM) * ((n + BN - 1) / BN);
   BZG_REQUIRE(tiles < (1L << 31), BZG_ERR_UNSUPPORTED, "gemm: too many tiles");
   dim3 grid((unsigned)tiles), block(kThreads);
-  if (vec)
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, BM, BN, WM, WN, true, TA, TB>), grid, block, 0, ctx->stream,
-                       m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-  else
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, BM, BN, WM, WN, false, TA, TB>), grid, block, 0, ctx->stream,
-                       m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  hipLaunchKernelGGL((gemm_mfma_kernel<T, BM, BN, WM, WN, BK, PF, TA, TB>), grid, block, 0, ctx->stream, m, n, k, alpha,
+                     A, lda, B, ldb, beta, C, ldc);
   BZG_LAUNCH_CHECK();
   return BZG_OK;
 }
@@ -488,13 +543,22 @@ TuneKey tune_key(int type, int64_t m, int64_t n, int64_t k) {
 template <typename T>
 constexpr int kShapes = sizeof(T) == 4 ? 4 : 3;
 
+// Tiles against the 256 CUs, from products of 64 .. 4096 rows and columns with k = 64, 300, 1500 (us,
+// FP64 / FP32).  A large tile reads less per flop but leaves CUs idle in its last round: 128 x 128
+// only from 960 tiles and with 92 % of the rounds' slots filled (4096^2, k = 4096: 2015 FP64 against
+// 2070 with 64 x 64; k = 1500, 3700^2, 841 tiles: 802 / 420 against 693 / 379; 2936^2, 529 tiles: 632 /
+// 326 against 457 / 253); FP32's 128 x 256 likewise from 480 tiles.  64 x 64 from 600 tiles (2000^2, k =
+// 1500: 249 / 137 against 291 / 171 with 32 x 32; 1500^2, 576 tiles: 190 / 103 against 169 / 103), and
+// from 200 for short k, where the loads ahead of the first product are most of the time (1000^2,
+// k = 64: 8.2 / 6.8 against 9.0 / 7.4).
 template <typename T>
-int heuristic_shape(int64_t m, int64_t n) {
-  if (sizeof(T) == 4 && ((m + 127) / 128) * ((n + 255) / 256) >= 240) return 3;
-  const long t128 = ((m + 127) / 128) * ((n + 127) / 128);
-  const long t64 = ((m + 63) / 64) * ((n + 63) / 64);
-  if (t128 >= 240) return 2;
-  if (t64 >= 200) return 1;
+int heuristic_shape(int64_t m, int64_t n, int64_t k) {
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+  auto filled = [](int64_t t) { return t * 100 >= 92 * ((t + 255) / 256 * 256); };
+  const int64_t t256 = tiles(128, 256), t128 = tiles(128, 128), t64 = tiles(64, 64);
+  if (sizeof(T) == 4 && t256 >= 480 && filled(t256)) return 3;
+  if (t128 >= 960 && filled(t128)) return 2;
+  if (t64 >= 600 || (t64 >= 200 && k <= (sizeof(T) == 8 ? 128 : 512))) return 1;
   return 0;
 }
 
@@ -503,13 +567,13 @@ bzg_status launch_shape_t(bzg_context* ctx, int shape, int64_t m, int64_t n, int
                           int64_t lda, const T* B, int64_t ldb, T beta, T* C, int64_t ldc) {
   if constexpr (sizeof(T) == 4) {
     if (shape == 3)
-      return launch_tile<T, 128, 256, 64, 128, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+      return launch_tile<T, 128, 256, 64, 128, 16, 1, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
   }
   if (shape == 2)
-    return launch_tile<T, 128, 128, 64, 64, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+    return launch_tile<T, 128, 128, 64, 64, 16, 1, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
   if (shape == 1)
-    return launch_tile<T, 64, 64, 32, 32, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-  return launch_tile<T, 32, 32, 16, 16, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+    return launch_tile<T, 64, 64, 32, 32, 128 / sizeof(T), 2, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  return launch_tile<T, 32, 32, 16, 16, 256 / sizeof(T), 2, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
 }
 
 template <typename T>
@@ -539,7 +603,7 @@ bzg_status gemm_dispatch(bzg_context* ctx, int64_t m, int64_t n, int64_t k, T al
     BZG_LAUNCH_CHECK();
     return BZG_OK;
   }
-  int shape = heuristic_shape<T>(m, n);
+  int shape = heuristic_shape<T>(m, n, k);
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune.find(tune_key(sizeof(T) == 8 ? 0 : 1, m, n, k));
