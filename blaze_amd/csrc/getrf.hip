@@ -38,33 +38,6 @@ constexpr int kPanel = 64;      // columns of a panel
 constexpr int kTrsmLeaf = 32;
 constexpr int64_t kMaxOrder = 32768;
 
-// v with the lanes permuted by a DPP control (a lane without a source keeps its own).
-template <int CTRL>
-__device__ __forceinline__ int dpp(int v) {
-  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
-}
-__device__ __forceinline__ int high_word(double v) { return (int)(__double_as_longlong(v) >> 32); }
-__device__ __forceinline__ unsigned low_word(double v) { return (unsigned)__double_as_longlong(v); }
-// v of lane l (uniform) in every lane's scalar copy
-__device__ __forceinline__ double lane_value(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane((int)low_word(v), l), hi = __builtin_amdgcn_readlane(high_word(v), l);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-// The lane of `among` with the largest v (v >= 0, or -1: no candidate), ties to the lowest pos.
-// `among` holds the lanes whose high words are largest: nearly always one lane, found by an integer
-// maximum (one DPP instruction a step, where the maximum of doubles takes seven).
-__device__ __forceinline__ int best_lane(unsigned long long among, double v, int pos) {
-  int src = __ffsll((long long)among) - 1;
-  for (among &= among - 1; among; among &= among - 1) {
-    const int o = __ffsll((long long)among) - 1;
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)low_word(v), o);
-    const unsigned ls = (unsigned)__builtin_amdgcn_readlane((int)low_word(v), src);
-    if (lo > ls || (lo == ls && __builtin_amdgcn_readlane(pos, o) < __builtin_amdgcn_readlane(pos, src))) src = o;
-  }
-  return src;
-}
-
 // Original position of what ends at position `pos` after the interchanges base + j <-> piv[j]
 // (j = 0 .. w - 1, in order): the interchanges followed backwards.
 __device__ __forceinline__ int swap_source(int pos, const int* piv, int base, int w) {

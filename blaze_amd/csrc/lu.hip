@@ -8,14 +8,14 @@
 // Execution model: a persistent grid (a few workgroups per CU) pulls system indices from an
 // atomic work counter in longest-first order, so uneven sizes (n = 1..512) balance without a
 // host round trip.  One workgroup of one wavefront (64 threads) owns one system at a time:
-//   factor: blocked right-looking LU, panel width 8 (FP64) or 16 (FP32).  The panel lives in
-//           the wavefront's registers (NM / 64 rows per lane); each column step is a per-lane
-//           argmax, a butterfly over the wavefront, the pivot row's broadcast and a rank-1
-//           update.  The panel's interchanges are then applied to the other columns in one
-//           gather (each lane follows the swaps backwards to find the source row of every
-//           touched position), the U12 block row is solved against the unit-lower L11, and the
-//           trailing matrix gets A22 -= L21 * U12 with MFMA 16x16x4 tiles (operands from LDS,
-//           A22 in place in HBM).
+//   factor: blocked right-looking LU, panel width 16 (FP64 beyond order 256: 8), two panels a
+//           block in FP64, one in FP32.  The panel lives in the wavefront's registers (NM / 64
+//           rows per lane); each column step is a per-lane argmax, its reduction over the
+//           wavefront, the pivot row's broadcast and a rank-1 update.  The block's interchanges
+//           are then applied to the other columns in one gather (each lane follows the swaps
+//           backwards to find the source row of every touched position), the U12 block row is
+//           solved against the unit-lower L11, and the trailing matrix gets A22 -= L21 * U12
+//           with MFMA 16x16x4 tiles (A22 in place in HBM).
 //   solve:  P*B is loaded into LDS; forward/backward substitution by 16-row blocks: the
 //           off-diagonal part is a dot product over the factored rows, the 16x16 diagonal block
 //           is solved by one lane per right-hand side.
@@ -36,11 +36,7 @@ namespace {
 
 constexpr int NT = 64;        // threads per workgroup: one wavefront per system
 constexpr int NW = NT / 64;   // wavefronts per workgroup
-constexpr int NB = 16;        // largest panel width
-// Panel width per precision: the panel lives in the registers of one wavefront (4 rows x
-// kNB values per lane), 8 doubles or 16 floats keep it at 64 registers.
-template <typename T>
-constexpr int kNB = sizeof(T) == 8 ? 8 : 16;
+constexpr int NB = 16;        // panel width of lu_factor (FP32): NM / 64 rows x NB values per lane in registers
 constexpr int NMAX = 512;     // largest system order
 constexpr int NSMALL = 256;   // systems up to this order use the NM = 256 kernels
 constexpr int RMAX = 8;       // largest number of right-hand sides
@@ -50,8 +46,8 @@ constexpr int UPAD = 16;      // row padding of the U12 buffer (conflict-free MF
 // the register panel (NM / 64 rows per lane).
 template <typename T, int NM>
 struct FactorShm {
-  T panel[NM][kNB<T> + 1];      // L11 / L21 of the current panel (rows beyond n are zero)
-  T ublk[kNB<T>][NM + UPAD];    // U12 of the current panel
+  T panel[NM][NB + 1];      // L11 / L21 of the current panel (rows beyond n are zero)
+  T ublk[NB][NM + UPAD];    // U12 of the current panel
 };
 
 template <typename T, int NM>
@@ -76,14 +72,6 @@ struct Misc {
 
 template <typename T>
 struct MfmaLU;
-template <>
-struct MfmaLU<double> {
-  using acc_t = d4;
-  __device__ static acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  __device__ static int row(int i, int lane) { return 4 * i + lane / 16; }
-};
 template <>
 struct MfmaLU<float> {
   using acc_t = f4;
@@ -115,7 +103,6 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
                          FactorShm<T, NM>& sh, Misc<NM>& misc) {
   using MF = MfmaLU<T>;
   using acc_t = typename MF::acc_t;
-  constexpr int NB = kNB<T>;
   constexpr int Q = NM / 64;  // panel rows per lane
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int info = 0;
@@ -367,6 +354,355 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
   return info;
 }
 
+template <int NM>
+struct Misc64 {
+  int perm[NM];               // row i of the factored system = original row perm[i]
+  int sys;
+};
+
+// ---- FP64 factorisation: two-level blocks ------------------------------------------------------
+// One wavefront factors the n x n row-major A in place, in blocks of OB = 2 NB columns made of two
+// register panels of NB columns.  The wavefronts of a CU work on different systems, whose trailing
+// matrices together exceed the L2, so the trailing matrix's traffic counts: it is read and written once
+// per 32 columns (orders up to 256).  Updated after every 8 columns it was four times that.  Beside
+// it, the wavefront waits: on memory between the phases and on the chain of a column step (2000 cycles).
+// So the orders up to 256 run two wavefronts a SIMD: 256 registers, LDS below 20 KB (U12 goes through
+// it 16 rows at a time, interchanged rows are gathered from memory and not staged in it).
+// 10,000 systems of orders 4..256, 1..8 right-hand sides, with their solves: 5.4 ms (11.5 ms with
+// panels of 8; 6.3 ms with one wavefront a SIMD).  With one, a wavefront's time was: tiles 19 %,
+// column steps 19 %, the solves 22 %, the second panel's update 9 %, U12 8 %, the rest loads and interchanges.
+// Every element is the same chain of fused multiply-adds, k ascending, whatever the blocking (an FP64
+// MFMA adds its four products one after another with one rounding each), so the factors do not
+// depend on it.
+template <int NM>
+struct FactorShm64 {
+  static constexpr int NB = NM > NSMALL ? 8 : 16;  // panel columns: NM / 64 rows x NB doubles per lane
+  static constexpr int OB = 2 * NB;
+  double ub[NB][72];          // U12 of up to 64 columns, NB rows at a time
+  double l11[OB][OB + 1];     // the block's unit lower triangle
+  int piv[OB];                // absolute pivot rows of the block
+  int src_top[OB];            // source row of each of the block's rows (beyond the block: its first row)
+  int low_dst[OB], low_src[OB];  // rows below that take part (-1: none) and their sources (else the first row)
+};
+
+// Column jj of the panel and then the columns after it (spelled out: the whole is longer than the
+// optimizer unrolls, and the register arrays need constant indices).
+template <int NM, int jj>
+__device__ __forceinline__ void panel_columns64(double (&P)[NM / 64][FactorShm64<NM>::NB], int (&lpos)[NM / 64], int m, int j0,
+                                                int nbe, int off, FactorShm64<NM>& sh, Misc64<NM>& misc, int& info) {
+  constexpr int NB = FactorShm64<NM>::NB, Q = NM / 64;
+  const int lane = threadIdx.x;
+  if (jj >= nbe) return;
+  double v = -1.0;
+  int r = 1 << 30, bq = 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    double a = (lpos[q] >= jj && lpos[q] < m) ? fabs(P[q][jj]) : -1.0;
+    if (a != a) a = -0.5;
+    if (a > v || (a == v && lpos[q] < r)) { v = a; r = lpos[q]; bq = q; }
+  }
+  const int key = v >= 0.0 ? high_word(v) : (v == -0.5 ? -1 : -2);
+  int k = key;
+  k = max(k, dpp<0x111>(k));  // row_shr:1, 2, 4, 8, row_bcast:15, 31: lane 63 has the maximum
+  k = max(k, dpp<0x112>(k));
+  k = max(k, dpp<0x114>(k));
+  k = max(k, dpp<0x118>(k));
+  k = max(k, dpp<0x142>(k));
+  k = max(k, dpp<0x143>(k));
+  k = __builtin_amdgcn_readlane(k, 63);
+  const int pl = best_lane(__ballot(key == k), v, r);
+  const int p = __builtin_amdgcn_readlane(r, pl);
+  const int pq = __builtin_amdgcn_readlane(bq, pl);
+  // the pivot row from column jj on, in scalar registers
+  double pr[NB];
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (pq == q) {
+#pragma unroll
+      for (int c = jj; c < NB; ++c) pr[c] = bcast(P[q][c], pl);
+    }
+  const double piv = pr[jj];
+  if (piv != 0.0) {
+    if (lane == 0) {
+      sh.piv[off + jj] = j0 + p;
+      const int t = misc.perm[j0 + jj];
+      misc.perm[j0 + jj] = misc.perm[j0 + p];
+      misc.perm[j0 + p] = t;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) lpos[q] = (lpos[q] == jj) ? p : ((lpos[q] == p) ? jj : lpos[q]);
+    const double rinv = 1.0 / piv;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      if (lpos[q] > jj && lpos[q] < m) {
+        const double l = P[q][jj] * rinv;
+        P[q][jj] = l;
+#pragma unroll
+        for (int c = jj + 1; c < NB; ++c) P[q][c] -= l * pr[c];
+      }
+    }
+  } else {
+    // exactly-zero pivot: no interchange, no scaling (dgetf2); the column below is zero
+    if (lane == 0) sh.piv[off + jj] = j0 + jj;
+    if (info == 0) info = j0 + jj + 1;
+  }
+  if constexpr (jj + 1 < NB) panel_columns64<NM, jj + 1>(P, lpos, m, j0, nbe, off, sh, misc, info);
+}
+
+// Factors columns j0 .. j0 + nbe - 1 on rows j0 .. n - 1 in registers: lane l holds the rows l, l + 64,
+// ... of the panel.  Rows never move between registers: each keeps its logical position (its row
+// index after the interchanges so far) and is written there at the end.  The pivot: the largest
+// |a|, a NaN below every number, ties to the lowest logical row; found as the largest high word
+// (integer DPP maxima) and, nearly always, the one lane that has it.  Pivots go to piv (absolute), the
+// panel's top rows to l11 from (off, off).  Returns the first exactly-zero pivot (1-based) or 0.
+template <int NM>
+__device__ __forceinline__ int factor_panel64(double* __restrict__ A, int n, int lda, int j0, int nbe, int off,
+                                              FactorShm64<NM>& sh, Misc64<NM>& misc) {
+  constexpr int NB = FactorShm64<NM>::NB;
+  constexpr int Q = NM / 64;
+  const int lane = threadIdx.x;
+  const int m = n - j0;
+  double P[Q][NB];
+  int lpos[Q];
+  int info = 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int rr = lane + 64 * q;
+    lpos[q] = (rr < m) ? rr : (1 << 20);  // rows beyond the matrix never become candidates
+    const double* row = A + (long)(j0 + rr) * lda + j0;
+    if (nbe == NB) {
+#pragma unroll
+      for (int c4 = 0; c4 < NB / 4; ++c4) {
+        dvec4u v = {0.0, 0.0, 0.0, 0.0};
+        if (rr < m) v = *reinterpret_cast<const dvec4u*>(row + 4 * c4);
+        P[q][4 * c4] = v[0]; P[q][4 * c4 + 1] = v[1]; P[q][4 * c4 + 2] = v[2]; P[q][4 * c4 + 3] = v[3];
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < NB; ++c) P[q][c] = (rr < m && c < nbe) ? row[c] : 0.0;
+    }
+  }
+  panel_columns64<NM, 0>(P, lpos, m, j0, nbe, off, sh, misc, info);
+  // each row at its final (logical) position
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (lane + 64 * q < m) {
+      const int lr = lpos[q];
+      double* row = A + (long)(j0 + lr) * lda + j0;
+      if (nbe == NB) {
+#pragma unroll
+        for (int c4 = 0; c4 < NB / 4; ++c4)
+          *reinterpret_cast<dvec4u*>(row + 4 * c4) =
+              dvec4u{P[q][4 * c4], P[q][4 * c4 + 1], P[q][4 * c4 + 2], P[q][4 * c4 + 3]};
+      } else {
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+          if (c < nbe) row[c] = P[q][c];
+      }
+      if (lr < nbe) {
+#pragma unroll
+        for (int c = 0; c < NB; ++c) sh.l11[off + lr][off + c] = P[q][c];
+      }
+    }
+  }
+  __syncthreads();
+  return info;
+}
+
+// Sources of every position that the interchanges base + j <-> piv[j] (j < w <= 32, in order) touch:
+// the interchanges followed backwards, lanes 0 .. 31 for the rows base + j, lanes 32 .. 63 for the pivot
+// rows below them.  Returns whether anything moves.
+template <int NM>
+__device__ __forceinline__ bool swap_lists64(FactorShm64<NM>& sh, int first, int base, int w) {
+  const int lane = threadIdx.x, q = lane & 31;
+  const int* piv = sh.piv + first;
+  int dst = -1;
+  if (q < w) dst = lane < 32 ? base + q : piv[q];
+  if (lane >= 32 && dst < base + w) dst = -1;
+  int pos = dst;
+  for (int j = w - 1; j >= 0; --j) {
+    const int pj = piv[j];
+    if (pos == base + j) pos = pj;
+    else if (pos == pj) pos = base + j;
+  }
+  if (q < FactorShm64<NM>::OB) {
+    if (lane < 32) {
+      sh.src_top[q] = dst >= 0 ? pos : base;
+    } else {
+      sh.low_dst[q] = dst;
+      sh.low_src[q] = dst >= 0 ? pos : base;
+    }
+  }
+  __syncthreads();
+  return __any(dst >= 0 && pos != dst);
+}
+
+// The interchanges in sh's lists on one column per lane: x[i] becomes the new value of row base + i, the
+// rows below are written (each receives a row of the block).  Every row is loaded once, all loads before
+// the first store.
+template <int NM, int K>
+__device__ __forceinline__ void gather_rows64(double* __restrict__ A, int lda, int base, unsigned col, bool on, bool moved,
+                                              const FactorShm64<NM>& sh, double (&x)[K]) {
+  if (!moved) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) x[i] = on ? (A + (long)(base + i) * lda)[col] : 0.0;
+    return;
+  }
+  double y[K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    const double* top = A + (long)__builtin_amdgcn_readfirstlane(sh.src_top[i]) * lda;
+    const double* low = A + (long)__builtin_amdgcn_readfirstlane(sh.low_src[i]) * lda;
+    x[i] = on ? top[col] : 0.0;
+    y[i] = on ? low[col] : 0.0;
+  }
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    const int dst = __builtin_amdgcn_readfirstlane(sh.low_dst[i]);
+    if (dst >= 0 && on) (A + (long)dst * lda)[col] = y[i];
+  }
+}
+
+// Only the interchanges of w <= K rows (columns whose L parts are final).
+template <int NM, int K>
+__device__ __forceinline__ void swap_columns64(double* __restrict__ A, int lda, int base, int w, int c_beg, int c_end,
+                                               FactorShm64<NM>& sh) {
+  for (int g0 = c_beg; g0 < c_end; g0 += 64) {
+    const unsigned col = g0 + (int)threadIdx.x;
+    const bool on = (int)col < c_end;
+    double x[K];
+    gather_rows64<NM, K>(A, lda, base, col, on, true, sh, x);
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+      if (on && i < w) (A + (long)(base + i) * lda)[col] = x[i];
+  }
+}
+
+// x := L11^-1 x, row i and then the rows after it.
+template <int i, int K, typename Shm>
+__device__ __forceinline__ void lower_solve64(double (&x)[K], const Shm& sh) {
+#pragma unroll
+  for (int k = 0; k < i; ++k) x[i] -= sh.l11[i][k] * x[k];
+  // L11 is read for every 64 columns anew, a row at a time: hoisted out of their loop, or held until a
+  // branch that uses x, its 496 entries would take twice the registers there are
+  __asm__ volatile("" : "+v"(x[i]) : : "memory");
+  if constexpr (i + 1 < K) lower_solve64<i + 1>(x, sh);
+}
+
+// Columns c_beg .. c_end - 1, 64 at a time, against the K factored columns jb .. jb + K - 1: the
+// interchanges, U12 = L11^-1 A12 (one column per lane), A22 -= L21 U12 by rows of CT 16 x 16 MFMA
+// tiles.  U12 of the columns stays in registers as MFMA operands; the next row of tiles and its
+// L21 rows are loaded while the current one is multiplied.
+template <int NM, int K, int CT>
+__device__ __forceinline__ void update_columns64(double* __restrict__ A, int n, int lda, int jb, int c_beg, int c_end,
+                                                 bool moved, FactorShm64<NM>& sh) {
+  constexpr int NB = FactorShm64<NM>::NB;
+  const int lane = threadIdx.x, r16 = lane & 15, g = lane >> 4;
+  for (int g0 = c_beg; g0 < c_end; g0 += 16 * CT) {
+    const unsigned col = g0 + lane;
+    const bool on = lane < 16 * CT && (int)col < c_end;
+    double b[CT][K / 4];
+    const int r0 = jb + K;
+    {
+      double x[K];
+      gather_rows64<NM, K>(A, lda, jb, col, on, moved, sh, x);
+      lower_solve64<1>(x, sh);
+#pragma unroll
+      for (int i = 0; i < K; ++i)
+        if (on) (A + (long)(jb + i) * lda)[col] = x[i];
+#pragma unroll
+      for (int h = 0; h < K; h += NB) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) sh.ub[i][lane] = x[h + i];
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+          for (int k = 0; k < NB / 4; ++k) b[t][h / 4 + k] = sh.ub[4 * k + g][16 * t + r16];
+        __syncthreads();
+      }
+    }
+    if (r0 < n) {
+      double a[K / 4], an[K / 4];
+      d4 acc[CT], next[CT];
+      auto load = [&](int r, double (&la)[K / 4], d4 (&lc)[CT]) __attribute__((always_inline)) {
+        const double* lrow = A + (long)min(r + r16, n - 1) * lda + jb + g;
+#pragma unroll
+        for (int k = 0; k < K / 4; ++k) la[k] = lrow[4 * k];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double* crow = A + (long)min(r + 4 * i + g, n - 1) * lda;
+#pragma unroll
+          for (int t = 0; t < CT; ++t) lc[t][i] = crow[min(g0 + 16 * t + r16, n - 1)];
+        }
+      };
+      load(r0, a, acc);
+      for (int r = r0; r < n; r += 16) {
+        load(r + 16 < n ? r + 16 : r0, an, next);
+#pragma unroll
+        for (int k = 0; k < K / 4; ++k)
+#pragma unroll
+          for (int t = 0; t < CT; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[k], b[t][k], acc[t], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int gr = r + 4 * i + g;
+#pragma unroll
+          for (int t = 0; t < CT; ++t) {
+            const int gc = g0 + 16 * t + r16;
+            if (gr < n && gc < c_end) A[(long)gr * lda + gc] = acc[t][i];
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < K / 4; ++k) a[k] = an[k];
+#pragma unroll
+        for (int t = 0; t < CT; ++t) acc[t] = next[t];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// LU factorisation of the n x n row-major matrix A (leading dimension lda) in place; as lu_factor.
+template <int NM>
+__device__ __forceinline__ int lu_factor64(double* __restrict__ A, int n, int lda, int32_t* __restrict__ ipiv,
+                                           FactorShm64<NM>& sh, Misc64<NM>& misc) {
+  constexpr int NB = FactorShm64<NM>::NB, OB = FactorShm64<NM>::OB;
+  const int tid = threadIdx.x;
+  int info = 0;
+  for (int i = tid; i < n; i += NT) misc.perm[i] = i;
+  __syncthreads();
+  for (int jb = 0; jb < n; jb += OB) {
+    const int ob = min(OB, n - jb), jend = jb + ob;
+    int f = factor_panel64<NM>(A, n, lda, jb, min(NB, ob), 0, sh, misc);
+    if (info == 0) info = f;
+    if (ob > NB) {
+      const int j1 = jb + NB, w1 = ob - NB;
+      bool mv = swap_lists64<NM>(sh, 0, jb, NB);
+      update_columns64<NM, NB, 1>(A, n, lda, jb, j1, jend, mv, sh);
+      f = factor_panel64<NM>(A, n, lda, j1, w1, NB, sh, misc);
+      if (info == 0) info = f;
+      // the second panel's interchanges on the first's columns, then L21 of the block into l11
+      if (swap_lists64<NM>(sh, NB, j1, w1)) {
+        swap_columns64<NM, NB>(A, lda, j1, w1, jb, j1, sh);
+        __syncthreads();
+      }
+      if (jend < n) {
+        for (int e = tid; e < NB * NB; e += NT) sh.l11[NB + e / NB][e % NB] = A[(long)(j1 + e / NB) * lda + jb + e % NB];
+        __syncthreads();
+      }
+    }
+    if (ipiv && tid < ob) ipiv[jb + tid] = sh.piv[tid] + 1;
+    // the block's interchanges on the columns on both sides (a partial block is the last: left only)
+    const bool mv = swap_lists64<NM>(sh, 0, jb, ob);
+    if (mv && jb > 0) {
+      swap_columns64<NM, OB>(A, lda, jb, ob, 0, jb, sh);
+      __syncthreads();
+    }
+    if (jend < n) update_columns64<NM, OB, 4>(A, n, lda, jb, jend, n, mv, sh);
+  }
+  return info;
+}
+
 // Dot products of up to 16 consecutive rows of M (row0 .. row0+nrows-1) with the columns of
 // the LDS matrix X (ld RMAX) over k in [kb, ke):  out(r, c) = sum_k M(row0+r, k) * X(k, c).
 // Thread t handles rows t/16 + 4j (j < 4) and k = kb + t%16 (mod 16): the loads of all 16
@@ -494,11 +830,11 @@ __device__ __forceinline__ void lu_solve(const T* __restrict__ LU, int n, int ld
   }
 }
 
-template <int NM>
-__device__ __forceinline__ int next_system(int* counter, Misc<NM>& misc) {
+template <typename Shm>
+__device__ __forceinline__ int next_system(int* counter, Shm& misc) {
   if (threadIdx.x == 0) misc.sys = atomicAdd(counter, 1);
   __syncthreads();
-  const int s = misc.sys;
+  const int s = __builtin_amdgcn_readfirstlane(misc.sys);  // uniform: so are the system's addresses
   __syncthreads();
   return s;
 }
@@ -511,7 +847,7 @@ __device__ __forceinline__ int next_system(int* counter, Misc<NM>& misc) {
 // the others; NM = NMAX: takes the systems listed in big_list (orders NSMALL+1 .. NMAX).
 // Systems outside 1..NMAX / 0..RMAX were marked info = -1 by classify_kernel.
 template <typename T, int NM>
-__global__ __launch_bounds__(NT) void gesv_batched_kernel(int count, const int32_t* __restrict__ nv,
+__global__ __launch_bounds__(NT, NM == NSMALL ? 2 : 1) void gesv_batched_kernel(int count, const int32_t* __restrict__ nv,
                                                           const int32_t* __restrict__ rv,
                                                           const int64_t* __restrict__ a_off,
                                                           const int64_t* __restrict__ b_off,
@@ -524,10 +860,10 @@ __global__ __launch_bounds__(NT) void gesv_batched_kernel(int count, const int32
                                                           const int* __restrict__ big_count,
                                                           int* counter, int mode) {
   __shared__ union {
-    FactorShm<T, NM> f;
-    SolveShm<T, NM> s;
+    FactorShm64<NM> f;
+    SolveShm<double, NM> s;
   } sh;
-  __shared__ Misc<NM> misc;
+  __shared__ Misc64<NM> misc;
   const int tid = threadIdx.x;
   if (NM != NSMALL) count = *big_count;
   for (;;) {
@@ -540,7 +876,7 @@ __global__ __launch_bounds__(NT) void gesv_batched_kernel(int count, const int32
     T* b = (mode != 1) ? B + b_off[s] : nullptr;
     int inf = 0;
     if (mode != 2) {
-      inf = lu_factor<T, NM>(a, n, n, ipiv ? ipiv + p_off[s] : nullptr, sh.f, misc);
+      inf = lu_factor64<NM>(a, n, n, ipiv ? ipiv + p_off[s] : nullptr, sh.f, misc);
     } else {
       // permutation from the pivots: the interchanges i <-> ipiv[i] - 1 in order
       if (tid == 0) {
@@ -737,17 +1073,17 @@ __global__ __launch_bounds__(NT) void dsgesv_batched_kernel(
 // workgroup's FP64 scratch, factor, solve B into X.  The NM = NSMALL instance takes the listed
 // systems of order <= NSMALL, the NM = NMAX instance the others (each skips the rest).
 template <int NM>
-__global__ __launch_bounds__(NT) void gesv_fallback_kernel(
+__global__ __launch_bounds__(NT, NM == NSMALL ? 2 : 1) void gesv_fallback_kernel(
     const int32_t* __restrict__ nv, const int32_t* __restrict__ rv,
     const int64_t* __restrict__ a_off, const int64_t* __restrict__ b_off,
     const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ X,
     int32_t* __restrict__ info, const int32_t* __restrict__ list, const int* list_count,
     int* counter, double* __restrict__ ws64) {
   __shared__ union {
-    FactorShm<double, NM> f;
+    FactorShm64<NM> f;
     SolveShm<double, NM> s;
   } sh;
-  __shared__ Misc<NM> misc;
+  __shared__ Misc64<NM> misc;
   const int tid = threadIdx.x;
   double* W = ws64 + (long)blockIdx.x * NM * NM;
   const int count = *list_count;
@@ -760,7 +1096,7 @@ __global__ __launch_bounds__(NT) void gesv_fallback_kernel(
     const double* a = A + a_off[s];
     for (int e = tid; e < n * n; e += NT) W[e] = a[e];
     __syncthreads();
-    const int inf = lu_factor<double, NM>(W, n, n, nullptr, sh.f, misc);
+    const int inf = lu_factor64<NM>(W, n, n, nullptr, sh.f, misc);
     if (tid == 0) info[s] = inf;
     if (inf == 0) {
       const double* b = B + b_off[s];
