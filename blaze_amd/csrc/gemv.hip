@@ -142,8 +142,7 @@ void launch_partials_reduce(bzg_context* ctx, int N, int P, T alpha, const T* pa
                      P, cw_log2, alpha, part, beta, y);
 }
 
-constexpr int kGemvTargetGroups = 2048;  // workgroups that keep every CU streaming
-constexpr int kGemvTTargetGroups = 4096;  // ... of the transposed form (4096: 152 us, 2048: 161 us, at 16384 x 12289 fp32)
+constexpr int kGemvTargetGroups = 2048;  // workgroups that keep every CU streaming (8 of 256 threads each)
 constexpr int kGemvMaxParts = 2048;      // partial sums per output entry
 
 template <typename T, int G, int R>
@@ -219,16 +218,17 @@ bzg_status gemv_dispatch(bzg_context* ctx, int64_t m, int64_t n, T alpha, const 
 // the column-major form of the product (TDMatDVecMultExpr).  Stage 1: a workgroup is CT
 // column threads by RL = 256 / CT row lanes; column thread c owns VW adjacent columns (one
 // 16-byte load per row, whatever the row's alignment), workgroup (cx, ry) covers columns
-// [cx CT VW, (cx + 1) CT VW) and, in row lane l, the rows ry CH + l + k RL of its chunk of CH
-// consecutive rows.  Bound by memory: 16384 x 12289 fp32 (rows of odd length, so no row but the
-// first is 16-byte aligned) runs in 149 us = 5.4 TB/s; with four 4-byte loads for such rows it was
-// 258 us, with rows dealt out round-robin instead of in chunks 155 us (aligned rows: 139 against
-// 154).  x[i] is the same for every column thread of a row lane.  Each thread keeps its column
+// [cx CT VW, (cx + 1) CT VW) and, in row lane l, every (grid y) RL-th row from ry RL + l, so that the
+// workgroups in flight read neighbouring rows.  Bound by memory: 16384 x 12289 fp32 (rows of odd
+// length, so no row but the first is 16-byte aligned) runs in 130 us = 6.2 TB/s; with four 4-byte
+// loads for such rows, and 2054 workgroups, it was 258 us.  A chunk of consecutive rows for each
+// workgroup was faster only with a grid that left its last round empty; at 16384 x 16384 fp64 it was
+// 315-336 us against 306.  x[i] is the same for every column thread of a row lane.  Each thread keeps its column
 // sums in row order; the RL row lanes are added in lane order through LDS and written to
 // part[ry][j].  Stage 2 adds the RY partials of column j in index order, so the result is
 // identical run to run.
 template <typename T>
-__global__ __launch_bounds__(256) void gemv_t_partial_kernel(int M, int N, const T* __restrict__ A, long lda,
+__global__ __launch_bounds__(256, 8) void gemv_t_partial_kernel(int M, int N, const T* __restrict__ A, long lda,
                                                              const T* __restrict__ x, T* __restrict__ part,
                                                              int ct_log2) {
   using AR = Arith<T>;
@@ -237,25 +237,27 @@ __global__ __launch_bounds__(256) void gemv_t_partial_kernel(int M, int N, const
   const int CT = 1 << ct_log2, RL = 256 >> ct_log2;
   const int ct = threadIdx.x & (CT - 1), rl = threadIdx.x >> ct_log2;
   const long j = ((long)blockIdx.x * CT + ct) * VW;
-  const long ch = ((M + gridDim.y - 1) / gridDim.y + RL - 1) / RL * RL;
-  const long i0 = (long)blockIdx.y * ch, i1 = min((long)M, i0 + ch);
+  // the last column thread of a row takes the row's last VW columns and drops those that are its
+  // neighbour's: a loop of its own for the remainder made small odd products 12-20 % slower
+  const long jc = N >= VW ? min(j, (long)N - VW) : j;
+  const long step = (long)gridDim.y * RL;
   T s[VW];
 #pragma unroll
   for (int e = 0; e < VW; ++e) s[e] = T(0);
   if (j < N) {
-    if (j + VW <= N) {
+    if (N >= VW) {
 #pragma unroll 8
-      for (long i = i0 + rl; i < i1; i += RL) {
+      for (long i = (long)blockIdx.y * RL + rl; i < M; i += step) {
         const T xi = x[i];
         T av[VW];
-        *reinterpret_cast<i4u*>(av) = __builtin_nontemporal_load(reinterpret_cast<const i4u*>(A + i * lda + j));
+        *reinterpret_cast<i4u*>(av) = __builtin_nontemporal_load(reinterpret_cast<const i4u*>(A + i * lda + jc));
 #pragma unroll
         for (int e = 0; e < VW; ++e) s[e] = AR::add(s[e], AR::mul(av[e], xi));
       }
     } else {
-      const int w = (int)min((long)VW, N - j);
+      const int w = N;
 #pragma unroll 4
-      for (long i = i0 + rl; i < i1; i += RL) {
+      for (long i = (long)blockIdx.y * RL + rl; i < M; i += step) {
         const T xi = x[i];
         const T* row = A + i * lda + j;
 #pragma unroll
@@ -277,7 +279,7 @@ __global__ __launch_bounds__(256) void gemv_t_partial_kernel(int M, int N, const
   if (rl == 0) {
 #pragma unroll
     for (int e = 0; e < VW; ++e)
-      if (j + e < N) part[(long)blockIdx.y * N + j + e] = s[e];
+      if (jc + e >= j && jc + e < N) part[(long)blockIdx.y * N + jc + e] = s[e];
   }
 }
 
@@ -303,9 +305,14 @@ bzg_status gemv_t_dispatch(bzg_context* ctx, int64_t m, int64_t n, T alpha, cons
   while (ct_log2 < 8 && ((int64_t)VW << ct_log2) < n) ++ct_log2;
   const int64_t ct = 1 << ct_log2, rl = 256 / ct;
   const int64_t cx = (n + ct * VW - 1) / (ct * VW);
-  // row partitions: enough workgroups to fill the chip, at least 16 rows per row lane
-  const int64_t ry = std::max<int64_t>(1, std::min<int64_t>({(int64_t)kGemvMaxParts, (m + 16 * rl - 1) / (16 * rl),
-                                                            (kGemvTTargetGroups + cx - 1) / cx}));
+  // row partitions: 16 rows or more per row lane, and the most workgroups that run all at once.  Rounded
+  // up instead, 24 x 86 = 2064 of them left a second round nearly empty (16384 x 12288: fp64 308 us
+  // against 230, fp32 161 against 124).  Few rows: 8 per row lane, one round of loads, while that
+  // leaves at most 256 partial sums (300 x 9001 fp64 13.7 us with 16, 11.4 with 8; 12000 x 1000
+  // fp32, 1500 sums: 19.4 and 22.8)
+  const int64_t rows = (m + rl - 1) / rl;
+  const int64_t want = std::max<int64_t>((rows + 15) / 16, std::min<int64_t>((rows + 7) / 8, 256));
+  const int64_t ry = std::max<int64_t>(1, std::min<int64_t>({(int64_t)kGemvMaxParts, want, kGemvTargetGroups / cx}));
   BZG_REQUIRE(cx < (1LL << 31), BZG_ERR_UNSUPPORTED, "gemv: too many columns");
   void* w = nullptr;
   bzg_status st = workspace(ctx, 11, (size_t)ry * n * sizeof(T), &w);
