@@ -239,11 +239,11 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
       }
     }
   };
-  auto multiply = [&](int buf) __attribute__((always_inline)) {
+  auto multiply_part = [&](auto kend, int buf) __attribute__((always_inline)) {
     const T* as = As[buf];
     const T* bs = Bs[buf];
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
+    for (int kk = 0; kk < decltype(kend)::value; kk += 4) {
       T a[FM], b[FN];
 #pragma unroll
       for (int i = 0; i < FM; ++i) a[i] = as[(wm0 + i * 16 + lane % 16) * LDA_S + kk + lane / 16];
@@ -255,6 +255,8 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
         for (int j = 0; j < FN; ++j) acc[i][j] = MF::mma(a[i], b[j], acc[i][j]);
     }
   };
+
+  auto multiply = [&](int buf) __attribute__((always_inline)) { multiply_part(std::integral_constant<int, BK>{}, buf); };
 
   constexpr std::true_type fast{};
   constexpr std::false_type any{};
@@ -292,17 +294,21 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
     }
     // Past the end slab 0 is requested again: with a conditional load the wait for slab kt + 1 could
     // not leave slab kt + 2 in flight.
-    for (; kt < nk; kt += 2) {
+    const int half = nk * BK - K >= BK / 2;
+    for (; kt < nk - half; kt += 2) {
       load_slab(any, kt + 2 < nk ? (kt + 2) * BK : 0, ra);
       multiply(0);
       if (kt + 1 < nk) store_slab(any, 1, (kt + 1) * BK, rb);
       __syncthreads();
-      if (kt + 1 >= nk) break;
+      if (kt + 1 >= nk - half) break;
       load_slab(any, kt + 3 < nk ? (kt + 3) * BK : 0, rb);
       multiply(1);
       if (kt + 2 < nk) store_slab(any, 0, (kt + 2) * BK, ra);
       __syncthreads();
     }
+    // a last slab of which at most half lies within K: the other half's products would be zeros
+    // (700 x 700, k = 333 FP32: 9.6 us, 10.3 with them; 412 x 346, k = 111 FP64: 5.0, 5.3)
+    if (half) multiply_part(std::integral_constant<int, BK / 2>{}, (nk - 1) & 1);
   }
 
   // Epilogue: C = alpha*acc + beta*C; beta == 0 never reads C (it may hold NaN/garbage).
