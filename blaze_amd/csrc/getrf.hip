@@ -645,7 +645,8 @@ __global__ __launch_bounds__(256) void trsm_leaf_kernel(const double* __restrict
 
 // ---- row permutation of the right-hand sides ---------------------------------------------------
 // For every 64 interchanges (one workgroup of 128 threads), the net move of the at most 128
-// positions they touch: move[128 b + t] = (destination, source), destination -1 for none.
+// positions they touch: move[128 b + t] = (destination, source), destination -1 for none.  Factors
+// from elsewhere may interchange a row with any other, also with one above its block.
 __global__ __launch_bounds__(128) void ipiv_moves_kernel(int n, const int32_t* __restrict__ ipiv,
                                                          int2* __restrict__ moves) {
   __shared__ int s_piv[kPanel];
@@ -655,7 +656,7 @@ __global__ __launch_bounds__(128) void ipiv_moves_kernel(int n, const int32_t* _
   const int q = t % kPanel;
   int dst = -1;
   if (q < w) dst = t < kPanel ? base + q : s_piv[q];
-  if (t >= kPanel && dst < base + w) dst = -1;
+  if (t >= kPanel && dst >= base && dst < base + w) dst = -1;
   moves[(long)blockIdx.x * 128 + t] = make_int2(dst, dst >= 0 ? swap_source(dst, s_piv, base, w) : -1);
 }
 
