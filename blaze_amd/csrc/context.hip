@@ -24,6 +24,7 @@ bzg_status workspace(bzg_context* ctx, int slot, size_t bytes, void** out) {
     hipError_t e = hipMalloc(&w.ptr, bytes);
     if (e != hipSuccess) {
       w.ptr = nullptr;
+      (void)hipGetLastError();  // reported here, not by the next launch's check
       set_error(std::string("workspace hipMalloc: ") + hipGetErrorString(e));
       return BZG_ERR_OUT_OF_MEMORY;
     }

@@ -974,11 +974,21 @@ bzg_status bzg_dgesv(bzg_context* ctx, int64_t n, int64_t nrhs, double* A, int64
   BZG_REQUIRE(nrhs >= 0 && ldb >= (nrhs > 0 ? nrhs : 1), BZG_ERR_INVALID_ARGUMENT, "dgesv: bad nrhs or ldb");
   if ((st = bzg_dgetrf(ctx, n, A, lda, ipiv, info))) return st;
   if (n == 0 || nrhs == 0) return BZG_OK;
-  BZG_REQUIRE(B != nullptr, BZG_ERR_INVALID_ARGUMENT, "dgesv: null B");
   // dgesv leaves B unchanged when the factorisation reports a zero pivot: the kernels that write B
   // read info on the device
-  bzg::ProfScope prof(ctx, "dgetrs");
-  return bzg::big::getrs_run(ctx, (int)n, (long)nrhs, A, (long)lda, ipiv, B, (long)ldb, false, info);
+  if (B != nullptr) {
+    bzg::ProfScope prof(ctx, "dgetrs");
+    st = bzg::big::getrs_run(ctx, (int)n, (long)nrhs, A, (long)lda, ipiv, B, (long)ldb, false, info);
+    if (st != BZG_ERR_OUT_OF_MEMORY) return st;
+  } else {
+    bzg::set_error("dgesv: null B");
+    st = BZG_ERR_INVALID_ARGUMENT;
+  }
+  // a singular matrix needs neither B nor the solve's scratch: only then is info read back
+  int32_t h_info = 0;
+  BZG_HIP_CHECK(hipMemcpyAsync(&h_info, info, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+  BZG_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+  return h_info != 0 ? BZG_OK : st;
 }
 
 bzg_status bzg_dgetri(bzg_context* ctx, int64_t n, double* A, int64_t lda, const int32_t* ipiv) {

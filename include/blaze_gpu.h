@@ -429,7 +429,8 @@ bzg_status bzg_dgetrs(bzg_context* ctx, int64_t n, int64_t nrhs, const double* A
                       const int32_t* ipiv, double* B, int64_t ldb);
 /* dgesv = dgetrf + dgetrs (replaces solve() for one system: blaze/math/dense/LSE.h:6343-6373 ->
  * solveNxN LSE.h:5229-5257 -> dgesv_, clapack/gesv.h:207).  B is left unchanged when info > 0
- * (decided on the device: the call does not synchronise). */
+ * (decided on the device: the call does not synchronise); such a call needs neither B nor scratch for
+ * the solve, so without them (B null, or no memory) info is read back: BZG_OK if it is set. */
 bzg_status bzg_dgesv(bzg_context* ctx, int64_t n, int64_t nrhs, double* A, int64_t lda, int32_t* ipiv,
                      double* B, int64_t ldb, int32_t* info);
 /* A := A^-1 from bzg_dgetrf's factors (info must have been 0): the inverse by LU of invert()
