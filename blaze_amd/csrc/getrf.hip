@@ -338,10 +338,12 @@ __global__ __launch_bounds__(256) void rank_update_kernel(double* __restrict__ A
 }
 
 // ---- 64-row triangular solves on LDS tiles ------------------------------------------------------
-// A 64 x 64 diagonal block of factors (padded to the identity) and the reciprocals of its diagonal.
+// A 64 x 64 diagonal block of factors (padded to the identity), the reciprocals of its diagonal and,
+// per wavefront that loaded it, whether it holds an infinity or a NaN.
 struct Diag64 {
   double l[kPanel][kPanel + 2];  // row stride 66: the MFMA operand reads hit 64 different banks
   double rinv[kPanel];
+  int special[4];
 };
 
 template <bool UPPER>
@@ -359,6 +361,15 @@ __device__ __forceinline__ void load_diag64(Diag64& d, const double* __restrict_
     d.l[r][c] = v[i];
     if (UPPER && r == c) d.rinv[r] = 1.0 / v[i];
   }
+  bool special = false;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) special |= !(fabs(v[i]) <= DBL_MAX);
+  special = __any(special);
+  if (c == 0) d.special[w] = special;
+}
+
+__device__ __forceinline__ bool has_special(const Diag64& d) {
+  return __builtin_amdgcn_readfirstlane(d.special[0] | d.special[1] | d.special[2] | d.special[3]) != 0;
 }
 
 // x / d from r = 1 / d: one correction step of the product, which rounds as the division does; the
@@ -387,12 +398,39 @@ __device__ __forceinline__ void substitute16(double (&x)[16], const Diag64& d, i
   }
 }
 
+// Rows 16 q .. 16 q + 15 of X minus T's columns 16 s .. 16 s + 15 times the solved part s, by one
+// wavefront.  FP64 MFMAs multiply a zero x(k) like any other; where the block holds an infinity or a NaN
+// that would make a NaN of a row that substitution never touches, so there the zeros are skipped.
+__device__ __forceinline__ void subtract_part16(double (*X)[16], const Diag64& d, int q, int s, bool special, int lane) {
+  const int r16 = lane & 15, g = lane >> 4;
+  d4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = X[16 * q + 4 * i + g][r16];
+  if (special) {
+#pragma unroll 1
+    for (int k = 0; k < 16; ++k) {
+      const double x = X[16 * s + k][r16];
+      if (x != 0.0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] -= x * d.l[16 * q + 4 * i + g][16 * s + k];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v = __builtin_amdgcn_mfma_f64_16x16x4f64(-d.l[16 * q + r16][16 * s + 4 * e + g], X[16 * s + 4 * e + g][r16], v, 0,
+                                               0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) X[16 * q + 4 * i + g][r16] = v[i];
+}
+
 // X (64 rows x 16 columns in LDS, row stride 16) := T^-1 X by one wavefront: 16 rows by substitution
-// (every 16-lane group alike; the first writes), their product subtracted from the remaining rows
-// with FP64 MFMAs.
+// (every 16-lane group alike; the first writes), their product subtracted from the remaining rows.
 template <bool UPPER>
 __device__ __forceinline__ void solve64_wave(double (*X)[16], const Diag64& d, int lane) {
   const int r16 = lane & 15, g = lane >> 4;
+  const bool special = has_special(d);
 #pragma unroll 1
   for (int s0 = 0; s0 < 4; ++s0) {
     const int s = UPPER ? 3 - s0 : s0;
@@ -407,17 +445,7 @@ __device__ __forceinline__ void solve64_wave(double (*X)[16], const Diag64& d, i
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
 #pragma unroll 1
-    for (int q = UPPER ? 0 : s + 1; q < (UPPER ? s : 4); ++q) {
-      d4 v;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = X[16 * q + 4 * i + g][r16];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v = __builtin_amdgcn_mfma_f64_16x16x4f64(-d.l[16 * q + r16][16 * s + 4 * e + g], X[16 * s + 4 * e + g][r16], v,
-                                                 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) X[16 * q + 4 * i + g][r16] = v[i];
-    }
+    for (int q = UPPER ? 0 : s + 1; q < (UPPER ? s : 4); ++q) subtract_part16(X, d, q, s, special, lane);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   }
 }
@@ -557,6 +585,7 @@ __global__ __launch_bounds__(256) void trsv_block_kernel(const double* __restric
     if (wr < rest1 && con) acc[i] = W[(long)wr * ldw + c0 + r16];
   }
   __syncthreads();
+  const bool special = has_special(s_d);
 #pragma unroll 1
   for (int s0 = 0; s0 < 4; ++s0) {
     const int s = UPPER ? 3 - s0 : s0;
@@ -573,15 +602,7 @@ __global__ __launch_bounds__(256) void trsv_block_kernel(const double* __restric
     }
     __syncthreads();
     if (UPPER ? wave < s : wave > s) {
-      d4 v;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = s_x[16 * wave + 4 * i + g][r16];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v = __builtin_amdgcn_mfma_f64_16x16x4f64(-s_d.l[16 * wave + r16][16 * s + 4 * e + g],
-                                                 s_x[16 * s + 4 * e + g][r16], v, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) s_x[16 * wave + 4 * i + g][r16] = v[i];
+      subtract_part16(s_x, s_d, wave, s, special, lane);
       // the wavefront that substitutes next reads, in each lane, what its other lanes wrote here
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     }
