@@ -361,11 +361,11 @@ __device__ __forceinline__ void load_diag64(Diag64& d, const double* __restrict_
     d.l[r][c] = v[i];
     if (UPPER && r == c) d.rinv[r] = 1.0 / v[i];
   }
-  bool special = false;
+  int top = 0;  // the largest exponent field
 #pragma unroll
-  for (int i = 0; i < 16; ++i) special |= !(fabs(v[i]) <= DBL_MAX);
-  special = __any(special);
-  if (c == 0) d.special[w] = special;
+  for (int i = 0; i < 16; ++i) top = max(top, high_word(v[i]) & 0x7ff00000);
+  top = __any(top == 0x7ff00000);
+  if (c == 0) d.special[w] = top;
 }
 
 __device__ __forceinline__ bool has_special(const Diag64& d) {
@@ -406,7 +406,7 @@ __device__ __forceinline__ void subtract_part16(double (*X)[16], const Diag64& d
   d4 v;
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] = X[16 * q + 4 * i + g][r16];
-  if (special) {
+  if (__builtin_expect(special, 0)) {
 #pragma unroll 1
     for (int k = 0; k < 16; ++k) {
       const double x = X[16 * s + k][r16];
