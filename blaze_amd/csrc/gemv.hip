@@ -38,7 +38,13 @@ struct Arith<int32_t> {  // wrap-around arithmetic, like the unsigned reinterpre
   }
 };
 
-template <typename T, int G, int R>
+template <bool NT, typename T>
+__device__ __forceinline__ i4u load16(const T* p) {
+  const i4u* q = reinterpret_cast<const i4u*>(p);
+  return NT ? __builtin_nontemporal_load(q) : *q;
+}
+
+template <typename T, int G, int R, bool NT>
 __global__ __launch_bounds__(256) void gemv_kernel(int M, int N, int KC, T alpha, const T* __restrict__ A,
                                                    long lda, const T* __restrict__ x, T beta,
                                                    T* __restrict__ y, T* __restrict__ part) {
@@ -58,6 +64,19 @@ __global__ __launch_bounds__(256) void gemv_kernel(int M, int N, int KC, T alpha
   for (int r = 0; r < R; ++r) acc[r] = T(0);
 
   const int vend = c1 / VW;  // c0 is a multiple of VW
+  // Tail columns (N not a multiple of VW).  Doubles read through the caches: the one there is is requested
+  // ahead of the vectors and added after them; a loop behind them waits for memory once more (100000 x
+  // 101: 14.9 us, 18.2).  The compiler then also requests both rows of a step before it waits, which
+  // gains as much again at such sizes (3000 x 3001: 13.7, 19.4) and costs 5 % at 16384 x 16384; the four
+  // rows of 4-byte types it does not.
+  constexpr bool TAIL_FIRST = sizeof(T) == 8 && !NT;
+  const long ct = (long)max(c0, vend * VW) + lane_in_group;
+  T xt = T(0), at[R];
+  if (TAIL_FIRST && lane_in_group == 0 && ct < c1) {
+    xt = x[ct];
+#pragma unroll
+    for (int r = 0; r < R; ++r) at[r] = row0 + r < M ? A[(row0 + r) * lda + ct] : T(0);
+  }
   for (int v = c0 / VW + lane_in_group; v < vend; v += G) {
     T xv[VW];
     *reinterpret_cast<i4u*>(xv) = *reinterpret_cast<const i4u*>(x + (long)v * VW);
@@ -65,19 +84,24 @@ __global__ __launch_bounds__(256) void gemv_kernel(int M, int N, int KC, T alpha
     for (int r = 0; r < R; ++r) {
       if (row0 + r < M) {
         T av[VW];
-        *reinterpret_cast<i4u*>(av) =
-            __builtin_nontemporal_load(reinterpret_cast<const i4u*>(A + (row0 + r) * lda + (long)v * VW));
+        *reinterpret_cast<i4u*>(av) = load16<NT>(A + (row0 + r) * lda + (long)v * VW);
 #pragma unroll
         for (int e = 0; e < VW; ++e) acc[r] = AR::add(acc[r], AR::mul(av[e], xv[e]));
       }
     }
   }
-  // tail columns (N not a multiple of VW)
-  for (int c = max(c0, vend * VW) + lane_in_group; c < c1; c += G) {
-    const T xc = x[c];
+  if (TAIL_FIRST) {
+    if (lane_in_group == 0 && ct < c1) {
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (row0 + r < M) acc[r] = AR::add(acc[r], AR::mul(A[(row0 + r) * lda + c], xc));
+      for (int r = 0; r < R; ++r) acc[r] = AR::add(acc[r], AR::mul(at[r], xt));
+    }
+  } else {
+    for (long c = ct; c < c1; c += G) {
+      const T xc = x[c];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (row0 + r < M) acc[r] = AR::add(acc[r], AR::mul(A[(row0 + r) * lda + c], xc));
+    }
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -145,6 +169,16 @@ void launch_partials_reduce(bzg_context* ctx, int N, int P, T alpha, const T* pa
 constexpr int kGemvTargetGroups = 2048;  // workgroups that keep every CU streaming (8 of 256 threads each)
 constexpr int kGemvMaxParts = 2048;      // partial sums per output entry
 
+// Whether A is read past the caches (non-temporal), as 4-byte types always are: large matrices gain
+// 5-15 %.  Doubles in rows of odd length lose by it while the 256 MB memory-side cache may hold the
+// matrix from the call before (5001 x 3001: 31.3 us, 19.5 through the caches, 22.1 with 8-byte loads
+// through them; transposed 29.8, 26.2, 26.1; read from memory 33.3, 24.6, 34.0 and 29.9, 29.8, 32.5).
+template <typename T>
+bool read_once(const T* A, int64_t m, int64_t lda) {
+  const bool aligned = (uintptr_t)A % 16 == 0 && lda * sizeof(T) % 16 == 0;
+  return aligned || (size_t)m * lda * sizeof(T) > (256u << 20);
+}
+
 template <typename T, int G, int R>
 bzg_status launch_gemv(bzg_context* ctx, int m, int n, T alpha, const T* A, long lda, const T* x,
                        T beta, T* y) {
@@ -173,8 +207,13 @@ bzg_status launch_gemv(bzg_context* ctx, int m, int n, T alpha, const T* A, long
     part = static_cast<T*>(w);
   }
   const dim3 grid((unsigned)blocks, (unsigned)ks);
-  hipLaunchKernelGGL((gemv_kernel<T, G, R>), grid, dim3(256), 0, ctx->stream, m, n, kc, alpha, A, lda, x, beta, y,
-                     part);
+  constexpr bool ALWAYS = sizeof(T) == 4;  // (one kernel only)
+  if (ALWAYS || read_once(A, m, lda))
+    hipLaunchKernelGGL((gemv_kernel<T, G, R, true>), grid, dim3(256), 0, ctx->stream, m, n, kc, alpha, A, lda, x, beta, y,
+                       part);
+  else
+    hipLaunchKernelGGL((gemv_kernel<T, G, R, ALWAYS>), grid, dim3(256), 0, ctx->stream, m, n, kc, alpha, A, lda, x, beta,
+                       y, part);
   if (ks > 1) launch_partials_reduce<T>(ctx, m, ks, alpha, part, beta, y);
   BZG_LAUNCH_CHECK();
   return BZG_OK;
@@ -227,7 +266,7 @@ bzg_status gemv_dispatch(bzg_context* ctx, int64_t m, int64_t n, T alpha, const 
 // sums in row order; the RL row lanes are added in lane order through LDS and written to
 // part[ry][j].  Stage 2 adds the RY partials of column j in index order, so the result is
 // identical run to run.
-template <typename T>
+template <typename T, bool NT>
 __global__ __launch_bounds__(256, 8) void gemv_t_partial_kernel(int M, int N, const T* __restrict__ A, long lda,
                                                              const T* __restrict__ x, T* __restrict__ part,
                                                              int ct_log2) {
@@ -250,7 +289,7 @@ __global__ __launch_bounds__(256, 8) void gemv_t_partial_kernel(int M, int N, co
       for (long i = (long)blockIdx.y * RL + rl; i < M; i += step) {
         const T xi = x[i];
         T av[VW];
-        *reinterpret_cast<i4u*>(av) = __builtin_nontemporal_load(reinterpret_cast<const i4u*>(A + i * lda + jc));
+        *reinterpret_cast<i4u*>(av) = load16<NT>(A + i * lda + jc);
 #pragma unroll
         for (int e = 0; e < VW; ++e) s[e] = AR::add(s[e], AR::mul(av[e], xi));
       }
@@ -309,9 +348,10 @@ bzg_status gemv_t_dispatch(bzg_context* ctx, int64_t m, int64_t n, T alpha, cons
   // up instead, 24 x 86 = 2064 of them left a second round nearly empty (16384 x 12288: fp64 308 us
   // against 230, fp32 161 against 124).  Few rows: 8 per row lane, one round of loads, while that
   // leaves at most 256 partial sums (300 x 9001 fp64 13.7 us with 16, 11.4 with 8; 12000 x 1000
-  // fp32, 1500 sums: 19.4 and 22.8)
+  // fp32, 1500 sums: 19.4 and 22.8) and 1536 workgroups (200 x 50000 fp64: 20.3 us with 1274, 22.4 with
+  // 1960; 3000 x 3000 fp64: 21.4 with 1128, 19.9 with 1536)
   const int64_t rows = (m + rl - 1) / rl;
-  const int64_t want = std::max<int64_t>((rows + 15) / 16, std::min<int64_t>((rows + 7) / 8, 256));
+  const int64_t want = std::max<int64_t>((rows + 15) / 16, std::min<int64_t>({(rows + 7) / 8, 256, 1536 / cx}));
   const int64_t ry = std::max<int64_t>(1, std::min<int64_t>({(int64_t)kGemvMaxParts, want, kGemvTargetGroups / cx}));
   BZG_REQUIRE(cx < (1LL << 31), BZG_ERR_UNSUPPORTED, "gemv: too many columns");
   void* w = nullptr;
@@ -319,8 +359,13 @@ bzg_status gemv_t_dispatch(bzg_context* ctx, int64_t m, int64_t n, T alpha, cons
   if (st) return st;
   T* part = static_cast<T*>(w);
   const dim3 grid((unsigned)cx, (unsigned)ry);
-  hipLaunchKernelGGL((gemv_t_partial_kernel<T>), grid, dim3(256), 0, ctx->stream, (int)m, (int)n, A, (long)lda, x,
-                     part, ct_log2);
+  constexpr bool ALWAYS = sizeof(T) == 4;
+  if (ALWAYS || read_once(A, m, lda))
+    hipLaunchKernelGGL((gemv_t_partial_kernel<T, true>), grid, dim3(256), 0, ctx->stream, (int)m, (int)n, A, (long)lda, x,
+                       part, ct_log2);
+  else
+    hipLaunchKernelGGL((gemv_t_partial_kernel<T, ALWAYS>), grid, dim3(256), 0, ctx->stream, (int)m, (int)n, A, (long)lda,
+                       x, part, ct_log2);
   launch_partials_reduce<T>(ctx, (int)n, (int)ry, alpha, part, beta, y);
   BZG_LAUNCH_CHECK();
   return BZG_OK;
