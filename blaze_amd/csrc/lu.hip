@@ -839,10 +839,8 @@ __device__ __forceinline__ int next_system(int* counter, Shm& misc) {
   return s;
 }
 
-// ---- plain FP64 (or FP32) dgesv / dgetrf / dgetrs: A and B in place ---------------------
+// ---- plain FP64 (or FP32) dgesv / dgetrf: A and B in place ------------------------------
 // MODE 0 (gesv): factor A, solve B.  MODE 1 (getrf): factor A only (rv may be null).
-// MODE 2 (getrs): A holds factors and ipiv its 1-based pivots (as written by MODE 1); the row
-// interchanges are applied to B in pivot order (LAPACK dlaswp) and B is solved in place.
 // NM = NSMALL: takes the systems of order <= NSMALL from the (ordered) index range and skips
 // the others; NM = NMAX: takes the systems listed in big_list (orders NSMALL+1 .. NMAX).
 // Systems outside 1..NMAX / 0..RMAX were marked info = -1 by classify_kernel.
@@ -874,25 +872,7 @@ __global__ __launch_bounds__(NT, NM == NSMALL ? 2 : 1) void gesv_batched_kernel(
     if (NM == NSMALL && (n < 1 || n > NSMALL || nrhs < 0 || nrhs > RMAX)) continue;
     T* a = A + a_off[s];
     T* b = (mode != 1) ? B + b_off[s] : nullptr;
-    int inf = 0;
-    if (mode != 2) {
-      inf = lu_factor64<NM>(a, n, n, ipiv ? ipiv + p_off[s] : nullptr, sh.f, misc);
-    } else {
-      // permutation from the pivots: the interchanges i <-> ipiv[i] - 1 in order
-      if (tid == 0) {
-        const int32_t* pv = ipiv + p_off[s];
-        for (int i = 0; i < n; ++i) misc.perm[i] = i;
-        for (int i = 0; i < n; ++i) {
-          const int q = pv[i] - 1;
-          if (q != i && q >= 0 && q < n) {
-            const int t = misc.perm[i];
-            misc.perm[i] = misc.perm[q];
-            misc.perm[q] = t;
-          }
-        }
-      }
-      __syncthreads();
-    }
+    const int inf = lu_factor64<NM>(a, n, n, ipiv ? ipiv + p_off[s] : nullptr, sh.f, misc);
     if (tid == 0 && info) info[s] = inf;
     if (inf == 0 && mode != 1) {
       for (int e = tid; e < n * RMAX; e += NT) {
@@ -903,6 +883,61 @@ __global__ __launch_bounds__(NT, NM == NSMALL ? 2 : 1) void gesv_batched_kernel(
       lu_solve<T>(a, n, n, sh.s.x, nrhs, sh.s.diag);
       for (int e = tid; e < n * nrhs; e += NT) b[e] = sh.s.x[(e / nrhs) * RMAX + e % nrhs];
     }
+    __syncthreads();
+  }
+}
+
+// dgetrs (MODE 2 of the launches below): LU holds factors and ipiv their 1-based pivots; the row interchanges
+// are applied to B in pivot order (LAPACK dlaswp) and B is solved in place.  Same work split as
+// gesv_batched_kernel.  W wavefronts a SIMD: two hide each other's waits but spill 69 registers, so a
+// batch that one a SIMD holds runs the other instance (1024 systems of order 256, one right-hand side: 300 us;
+// 1100 of them, two a SIMD: 369).  A kernel of its own: as a mode of gesv_batched_kernel, whose
+// registers the factorisation decides, these took 387 and 424.
+template <int NM, int W>
+__global__ __launch_bounds__(NT, W) void getrs_batched_kernel(int count, const int32_t* __restrict__ nv,
+                                                              const int32_t* __restrict__ rv,
+                                                              const int64_t* __restrict__ a_off,
+                                                              const int64_t* __restrict__ b_off,
+                                                              const int64_t* __restrict__ p_off,
+                                                              const double* __restrict__ LU, double* __restrict__ B,
+                                                              const int32_t* __restrict__ ipiv,
+                                                              int32_t* __restrict__ info,
+                                                              const int32_t* __restrict__ order,
+                                                              const int32_t* __restrict__ big_list,
+                                                              const int* __restrict__ big_count, int* counter) {
+  __shared__ SolveShm<double, NM> sh;
+  __shared__ Misc64<NM> misc;
+  const int tid = threadIdx.x;
+  if (NM != NSMALL) count = *big_count;
+  for (;;) {
+    const int idx = next_system(counter, misc);
+    if (idx >= count) break;
+    const int s = (NM != NSMALL) ? big_list[idx] : (order ? order[idx] : idx);
+    const int n = nv[s], nrhs = rv ? rv[s] : 0;
+    if (NM == NSMALL && (n < 1 || n > NSMALL || nrhs < 0 || nrhs > RMAX)) continue;
+    double* b = B + b_off[s];
+    // permutation from the pivots: the interchanges i <-> ipiv[i] - 1 in order
+    if (tid == 0) {
+      const int32_t* pv = ipiv + p_off[s];
+      for (int i = 0; i < n; ++i) misc.perm[i] = i;
+      for (int i = 0; i < n; ++i) {
+        const int q = pv[i] - 1;
+        if (q != i && q >= 0 && q < n) {
+          const int t = misc.perm[i];
+          misc.perm[i] = misc.perm[q];
+          misc.perm[q] = t;
+        }
+      }
+    }
+    __syncthreads();
+    for (int e = tid; e < n * RMAX; e += NT) {
+      const int i = e / RMAX, c = e % RMAX;
+      sh.x[e] = (c < nrhs) ? b[(long)misc.perm[i] * nrhs + c] : 0.0;
+    }
+    __syncthreads();
+    lu_solve<double>(LU + a_off[s], n, n, sh.x, nrhs, sh.diag);
+    for (int e = tid; e < n * nrhs; e += NT) b[e] = sh.x[(e / nrhs) * RMAX + e % nrhs];
+    if (tid == 0 && info) info[s] = 0;
     __syncthreads();
   }
 }
@@ -1222,7 +1257,7 @@ bzg_status bzg_batched_order(bzg_context* ctx, int64_t count, const int32_t* n_h
 
 namespace bzg {
 namespace {
-// Batched LU entry points (MODE as in gesv_batched_kernel).
+// Batched LU entry points (mode 0 gesv, 1 getrf, 2 getrs).
 // Scratch of one call: counters[0] small-kernel work counter, [1] big count, [2] big-kernel
 // work counter (at least 8 ints, cleared by a kernel); big = room for `count` system indices
 // (the systems of order > NSMALL).  Allocates nothing.
@@ -1238,15 +1273,27 @@ bzg_status lu_batched_scratch(bzg_context* ctx, int mode, int64_t count, const i
   // the few systems of order > NSMALL first (their kernel holds 2 workgroups per CU), then
   // the rest at full occupancy; persistent grids never larger than the batch
   const int64_t cap = std::max<int64_t>(count, 1);
-  hipLaunchKernelGGL((gesv_batched_kernel<double, NMAX>),
-                     dim3((unsigned)std::min<int64_t>(ctx->num_cus * 2, cap)), dim3(NT), 0,
-                     ctx->stream, (int)count, n, nrhs, a_off, b_off, p_off, A, B, ipiv, info, order,
-                     (const int32_t*)big, (const int*)(counters + 1), counters + 2, mode);
-  BZG_LAUNCH_CHECK();
-  const int grid = (int)std::min<int64_t>(ctx->num_cus * g_tuning.wg_per_cu_fp64, cap);
-  hipLaunchKernelGGL((gesv_batched_kernel<double, NSMALL>), dim3(grid), dim3(NT), 0,
-                     ctx->stream, (int)count, n, nrhs, a_off, b_off, p_off, A, B, ipiv, info, order,
-                     (const int32_t*)big, (const int*)(counters + 1), counters + 0, mode);
+  const dim3 grid_big((unsigned)std::min<int64_t>(ctx->num_cus * 2, cap));
+  const dim3 grid((unsigned)std::min<int64_t>(ctx->num_cus * g_tuning.wg_per_cu_fp64, cap));
+  const int32_t* list = big;
+  const int* list_count = counters + 1;
+  if (mode == 2) {
+    hipLaunchKernelGGL((getrs_batched_kernel<NMAX, 1>), grid_big, dim3(NT), 0, ctx->stream, (int)count, n, nrhs, a_off,
+                       b_off, p_off, A, B, ipiv, info, order, list, list_count, counters + 2);
+    BZG_LAUNCH_CHECK();
+    if (count <= ctx->num_cus * 4)
+      hipLaunchKernelGGL((getrs_batched_kernel<NSMALL, 1>), grid, dim3(NT), 0, ctx->stream, (int)count, n, nrhs, a_off,
+                         b_off, p_off, A, B, ipiv, info, order, list, list_count, counters + 0);
+    else
+      hipLaunchKernelGGL((getrs_batched_kernel<NSMALL, 2>), grid, dim3(NT), 0, ctx->stream, (int)count, n, nrhs, a_off,
+                         b_off, p_off, A, B, ipiv, info, order, list, list_count, counters + 0);
+  } else {
+    hipLaunchKernelGGL((gesv_batched_kernel<double, NMAX>), grid_big, dim3(NT), 0, ctx->stream, (int)count, n, nrhs,
+                       a_off, b_off, p_off, A, B, ipiv, info, order, list, list_count, counters + 2, mode);
+    BZG_LAUNCH_CHECK();
+    hipLaunchKernelGGL((gesv_batched_kernel<double, NSMALL>), grid, dim3(NT), 0, ctx->stream, (int)count, n, nrhs, a_off,
+                       b_off, p_off, A, B, ipiv, info, order, list, list_count, counters + 0, mode);
+  }
   BZG_LAUNCH_CHECK();
   return BZG_OK;
 }
