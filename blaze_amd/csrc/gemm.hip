@@ -268,11 +268,14 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
   store_slab(any, 0, 0, ra);
   __syncthreads();
   int kt = 0;
+  // A last slab of which at most half lies within K: the other half's products would be zeros (700 x 700,
+  // k = 333 FP32: 9.6 us, 10.3 with them; 412 x 346, k = 111 FP64: 5.0, 5.3).  Large tiles are for long K.
+  const int half = BM <= 64 && nk * BK - K >= BK / 2;
   if (PF == 1) {
     // Past the end slab 0 is requested again: with the last load left out by a branch 4096^3 FP64
     // takes 2.14 ms instead of 2.02 (and 2.11 as one basic block, where the compiler moves the loads
     // down between the products).
-    for (; kt < nk; ++kt) {
+    for (; kt < nk - half; ++kt) {
       load_slab(any, kt + 1 < nk ? (kt + 1) * BK : 0, ra);
       multiply(kt & 1);
       if (kt + 1 < nk) store_slab(any, (kt & 1) ^ 1, (kt + 1) * BK, ra);
@@ -294,7 +297,6 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
     }
     // Past the end slab 0 is requested again: with a conditional load the wait for slab kt + 1 could
     // not leave slab kt + 2 in flight.
-    const int half = nk * BK - K >= BK / 2;
     for (; kt < nk - half; kt += 2) {
       load_slab(any, kt + 2 < nk ? (kt + 2) * BK : 0, ra);
       multiply(0);
@@ -306,10 +308,8 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
       if (kt + 2 < nk) store_slab(any, 0, (kt + 2) * BK, ra);
       __syncthreads();
     }
-    // a last slab of which at most half lies within K: the other half's products would be zeros
-    // (700 x 700, k = 333 FP32: 9.6 us, 10.3 with them; 412 x 346, k = 111 FP64: 5.0, 5.3)
-    if (half) multiply_part(std::integral_constant<int, BK / 2>{}, (nk - 1) & 1);
   }
+  if (half) multiply_part(std::integral_constant<int, BK / 2>{}, (nk - 1) & 1);
 
   // Epilogue: C = alpha*acc + beta*C; beta == 0 never reads C (it may hold NaN/garbage).
   const bool read_c = beta != T(0);
@@ -345,7 +345,11 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(int M, int N, in
 }
 
 // ---- grouped GEMM: many independent products of uneven sizes in one persistent launch ----
-constexpr int kGT = 64;  // tile of the grouped kernel (64 x 64, waves of 32 x 32)
+// Tile of the grouped kernel: 64 x 64, waves of 32 x 32, one shallow slab ahead.  Its workgroups go from
+// tile to tile, four to a CU, so the others' products cover a tile's first loads, and the deeper
+// prefetch that a small single product needs costs more than it hides (3000 products of 16..100: 137 us, 171
+// with two slabs ahead, 174 with slabs of 32).
+constexpr int kGT = 64;
 constexpr int kGBK = 16;
 
 // Tiles of one problem; a problem that fails the bzg_dgemm argument rules gets none (and
@@ -415,7 +419,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_grouped_kernel(int count, co
         }
       }
     } else {
-      gemm_tile<double, kGT, kGT, 32, 32, kGBK, 2>((int)q.m, (int)q.n, (int)q.k, q.alpha, q.A, q.lda, q.B, q.ldb,
+      gemm_tile<double, kGT, kGT, 32, 32, kGBK, 1>((int)q.m, (int)q.n, (int)q.k, q.alpha, q.A, q.lda, q.B, q.ldb,
                                                    q.beta, q.C, q.ldc, tm, tn, sh);
     }
     __syncthreads();  // LDS of this tile is free before the next one is staged
