@@ -176,7 +176,10 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
       for (int e = 0; e < VW; ++e) v[e] = p[min(col + e, cmax)];
     }
   };
-  // `fast`: the slab is full and both operands are read by vectors, known at compile time
+  // `fast`: the slab is full and both operands are read by vectors, known at compile time.  SHALLOW tiles
+  // often have no other slab than a partial one: where its rows run along k, those past K are read as the
+  // last one, by vectors (3000 x 1000, k = 10 FP32, A transposed: 6.6 us, 7.3).
+  constexpr bool SHALLOW = BM == 64 && PF == 1;
   auto load_slab = [&](auto fast, int k0, Regs& r) __attribute__((always_inline)) {
     constexpr bool FAST = decltype(fast)::value;
     const bool kfull = k0 + BK <= K;
@@ -186,6 +189,11 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
       for (int i = 0; i < NA; ++i)
         load_op(std::integral_constant<bool, TA>{}, true, A, lda, m0, M, k0, tid / A_VPR + i * A_RPP, (tid % A_VPR) * VW,
                 r.a[i]);
+    } else if (SHALLOW && TA && vec_a) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+        load_op(std::integral_constant<bool, TA>{}, true, A, lda, m0, M, k0, min(tid / A_VPR + i * A_RPP, K - 1 - k0),
+                (tid % A_VPR) * VW, r.a[i]);
     } else {
 #pragma unroll
       for (int i = 0; i < NA; ++i)
@@ -196,6 +204,11 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
 #pragma unroll
       for (int i = 0; i < NB; ++i)
         load_op(std::integral_constant<bool, !TB>{}, true, B, ldb, n0, N, k0, tid / B_VPR + i * B_RPP,
+                (tid % B_VPR) * VW, r.b[i]);
+    } else if (SHALLOW && !TB && vec_b) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+        load_op(std::integral_constant<bool, !TB>{}, true, B, ldb, n0, N, k0, min(tid / B_VPR + i * B_RPP, K - 1 - k0),
                 (tid % B_VPR) * VW, r.b[i]);
     } else {
 #pragma unroll
@@ -552,6 +565,7 @@ TuneKey tune_key(int type, int64_t m, int64_t n, int64_t k) {
 // 8192^3, 112.0 against 102.7 at 4096^3.
 template <typename T>
 constexpr int kShapes = sizeof(T) == 4 ? 4 : 3;
+constexpr int kShortK = 4;  // FP32 only, by rule: 64x64 with slabs of 16 and one ahead, as in the grouped kernel
 
 // Tiles against the 256 CUs, from products of 64 .. 4096 rows and columns with k = 64, 300, 1500 (us,
 // FP64 / FP32).  A large tile reads less per flop but leaves CUs idle in its last round: 128 x 128
@@ -560,7 +574,9 @@ constexpr int kShapes = sizeof(T) == 4 ? 4 : 3;
 // 326 against 457 / 253); FP32's 128 x 256 likewise from 480 tiles.  64 x 64 from 600 tiles (2000^2, k =
 // 1500: 249 / 137 against 291 / 171 with 32 x 32; 1500^2, 576 tiles: 190 / 103 against 169 / 103), and
 // from 200 for short k, where the loads ahead of the first product are most of the time (1000^2,
-// k = 64: 8.2 / 6.8 against 9.0 / 7.4).
+// k = 64: 8.2 / 6.8 against 9.0 / 7.4).  FP32 up to k = 64 with shallow slabs, which leave less of the last one
+// outside K (1500^2, k = 20: 6.3 us, 8.8 with slabs of 32, both operands transposed 6.5, 9.1; 2000^2, k = 48:
+// 9.6, 10.8; 1200^2, k = 64: 7.0, 7.5); from k = 100 the deep ones are ahead (1000^2: 7.3).
 template <typename T>
 int heuristic_shape(int64_t m, int64_t n, int64_t k) {
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
@@ -568,6 +584,7 @@ int heuristic_shape(int64_t m, int64_t n, int64_t k) {
   const int64_t t256 = tiles(128, 256), t128 = tiles(128, 128), t64 = tiles(64, 64);
   if (sizeof(T) == 4 && t256 >= 480 && filled(t256)) return 3;
   if (t128 >= 960 && filled(t128)) return 2;
+  if (sizeof(T) == 4 && t64 >= 200 && k <= 64) return kShortK;
   if (t64 >= 600 || (t64 >= 200 && k <= (sizeof(T) == 8 ? 128 : 512))) return 1;
   return 0;
 }
@@ -578,6 +595,10 @@ bzg_status launch_shape_t(bzg_context* ctx, int shape, int64_t m, int64_t n, int
   if constexpr (sizeof(T) == 4) {
     if (shape == 3)
       return launch_tile<T, 128, 256, 64, 128, 16, 1, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (shape == kShortK)
+      return launch_tile<T, 64, 64, 32, 32, 16, 1, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
   }
   if (shape == 2)
     return launch_tile<T, 128, 128, 64, 64, 16, 1, TA, TB>(ctx, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
