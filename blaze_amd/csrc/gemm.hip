@@ -144,8 +144,12 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
   const int wm0 = (wave / WAVES_N) * WM;
   const int wn0 = (wave % WAVES_N) * WN;
 
-  const int m0 = tm * BM;
-  const int n0 = tn * BN;
+  // Where an operand's stored rows run along m (A transposed) or n (B not), the matrix's last tile starts early
+  // enough to be whole and stores only what its neighbour does not: all its loads stay vectors.  Read
+  // element by element, such tiles were the last to end (2000^3 FP64, A transposed: 349 us, 259; 1000^3
+  // FP32: 41.3, 29.6; 412 x 346, k = 111 FP32: 5.2, 4.6).
+  const int m0 = TA && M >= BM ? min(tm * BM, M - BM) : tm * BM;
+  const int n0 = !TB && N >= BN ? min(tn * BN, N - BN) : tn * BN;
 
   acc_t acc[FM][FN];
 #pragma unroll
@@ -334,7 +338,7 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, T alpha, const T*
       for (int r = 0; r < 4; ++r) {
         const int gr = m0 + wm0 + i * 16 + MF::row(r, lane);
         const int gc = n0 + wn0 + j * 16 + lane % 16;
-        if (gr < M && gc < N) {
+        if (gr < M && gc < N && (!TA || gr >= tm * BM) && (TB || gc >= tn * BN)) {
           T* p = C + (long)gr * ldc + gc;
           T v = alpha * acc[i][j][r];
           if (read_c) v += beta * *p;
