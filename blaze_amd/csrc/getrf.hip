@@ -704,6 +704,16 @@ __global__ __launch_bounds__(128) void moves_to_perm_kernel(int n, const int2* _
   for (int i = t; i < n; i += 128) perm[i] = sp[i];
 }
 
+// perm of up to 64 interchanges in one launch: each position traced back by itself.
+__global__ __launch_bounds__(64) void ipiv_to_perm64_kernel(int n, const int32_t* __restrict__ ipiv,
+                                                            int32_t* __restrict__ perm) {
+  __shared__ int s_piv[kPanel];
+  const int t = threadIdx.x;
+  s_piv[t] = t < n ? ipiv[t] - 1 : t;
+  __syncthreads();
+  if (t < n) perm[t] = swap_source(t, s_piv, 0, n);
+}
+
 // W[i][c] = B[perm[i]][c] (identity = true: W = P I, the permuted identity, n x n)
 __global__ __launch_bounds__(256) void gather_rows_kernel(int n, long ncols, const int32_t* __restrict__ perm,
                                                           const double* __restrict__ B, long ldb,
@@ -746,11 +756,13 @@ __global__ void det_kernel(int n, const double* __restrict__ A, long lda, const 
 
 // ---- host side -------------------------------------------------------------------------------
 // threads, rows per thread and leaf width for a panel of m rows: one wavefront per SIMD while its
-// registers hold 16 columns of the block, then two, then fewer columns
+// registers hold 16 columns of the block, then two, then fewer columns.  The smallest matrices (and a last
+// panel's end) take half the column loop: n = 1 10.8 us, 15.3 with the 16-column leaf; n = 8 13.0, 20.6.
 struct LeafShape {
   int t, r, wl;
 };
 static LeafShape leaf_shape(int64_t m) {
+  if (m <= 8) return {256, 1, 8};
   static const LeafShape shapes[] = {{256, 1, 16}, {256, 2, 16}, {256, 4, 16}, {256, 6, 16}, {512, 4, 16},
                                      {512, 6, 12}, {512, 8, 8},  {512, 16, 4}, {512, 32, 2}, {512, 64, 1}};
   for (const LeafShape& s : shapes)
@@ -766,7 +778,7 @@ static bzg_status launch_leaf(bzg_context* ctx, double* A, long lda, int n, int 
   const int r0 = c0 + w, nc = p0 + nbp - r0, rows = n - r0;
   const unsigned ugrid = (unsigned)((rows + 4 * kRankRows - 1) / (4 * kRankRows));
 #define BZG_LEAF(TT, RR, WW)                                                                               \
-  if (sh.t == TT && sh.r == RR) {                                                                          \
+  if (sh.t == TT && sh.r == RR && sh.wl == WW) {                                                           \
     hipLaunchKernelGGL((getf2_leaf_kernel<TT, RR, WW>), dim3(1), dim3(TT), 0, ctx->stream, A, lda, n, c0, w, p0, nbp, \
                        ipiv, info);                                                                        \
     BZG_LAUNCH_CHECK();                                                                                    \
@@ -776,6 +788,7 @@ static bzg_status launch_leaf(bzg_context* ctx, double* A, long lda, int n, int 
     }                                                                                                      \
     return BZG_OK;                                                                                         \
   }
+  BZG_LEAF(256, 1, 8)
   BZG_LEAF(256, 1, 16)
   BZG_LEAF(256, 2, 16)
   BZG_LEAF(256, 4, 16)
@@ -908,15 +921,18 @@ static bzg_status perm_attr(bzg_context* ctx) {
 }
 
 // Right-hand sides up to which a triangular solve runs block by block (trsv_block_kernel); more
-// go through the recursion and bzg_dgemm.
+// go through the recursion and bzg_dgemm, and so do matrices with fewer rows than this: there a thread
+// solves a column by itself (n = 12, 16 right-hand sides: 20.8 us, 22.7 by blocks; 20, 17: 24.6, 27.1; alike
+// at 24).
 constexpr long kBlockSolveCols = 64;
+constexpr int kBlockSolveRows = 25;
 
 // B := A^-1 B (B := A^-1 when identity) from the factors, unless info is given and nonzero:
 // W = P B (or P I) in the context's workspaces, forward and back substitution.
 static bzg_status getrs_run(bzg_context* ctx, int n, long ncols, const double* LU, long lda, const int32_t* ipiv,
                             double* B, long ldb, bool identity, const int32_t* info) {
   // (the inverse replaces the factors, which the block solve still reads when it writes B)
-  const bool blocks = !identity && ncols <= kBlockSolveCols;
+  const bool blocks = !identity && ncols <= kBlockSolveCols && n >= kBlockSolveRows;
   const int nblk = (n + kPanel - 1) / kPanel;
   // slot 13: the interchanges' moves and perm; slot 14: W and, for the block solve, the forward
   // solution
@@ -928,10 +944,15 @@ static bzg_status getrs_run(bzg_context* ctx, int n, long ncols, const double* L
   int2* moves = static_cast<int2*>(p);
   int32_t* perm = reinterpret_cast<int32_t*>(moves + (size_t)nblk * 128);
   double* W = static_cast<double*>(w);
-  hipLaunchKernelGGL(ipiv_moves_kernel, dim3((unsigned)nblk), dim3(128), 0, ctx->stream, n, ipiv, moves);
-  BZG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(moves_to_perm_kernel, dim3(1), dim3(128), (size_t)n * sizeof(int), ctx->stream, n, moves, perm);
-  BZG_LAUNCH_CHECK();
+  if (nblk == 1) {  // (a launch less: n = 12, 65 right-hand sides 20.9 us, 24.1)
+    hipLaunchKernelGGL(ipiv_to_perm64_kernel, dim3(1), dim3(64), 0, ctx->stream, n, ipiv, perm);
+    BZG_LAUNCH_CHECK();
+  } else {
+    hipLaunchKernelGGL(ipiv_moves_kernel, dim3((unsigned)nblk), dim3(128), 0, ctx->stream, n, ipiv, moves);
+    BZG_LAUNCH_CHECK();
+    hipLaunchKernelGGL(moves_to_perm_kernel, dim3(1), dim3(128), (size_t)n * sizeof(int), ctx->stream, n, moves, perm);
+    BZG_LAUNCH_CHECK();
+  }
   const long total = (long)n * ncols;
   hipLaunchKernelGGL(gather_rows_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, n, ncols,
                      perm, B, ldb, W, ncols, identity);
