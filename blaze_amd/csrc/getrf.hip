@@ -372,8 +372,11 @@ __device__ __forceinline__ bool has_special(const Diag64& d) {
   return __builtin_amdgcn_readfirstlane(d.special[0] | d.special[1] | d.special[2] | d.special[3]) != 0;
 }
 
-// x / d from r = 1 / d: one correction step of the product, which rounds as the division does; the
-// division itself where the product or its remainder may leave the range of normal numbers.
+// x / d from r = 1 / d, which is off the column's chain: the product and one correction by its remainder
+// (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", IBM J.
+// Res. Dev. 34, 1990: with r correctly rounded and the product within an ulp, the corrected quotient is
+// the rounded one); the division itself where the product or its remainder may leave the range of
+// normal numbers.
 __device__ __forceinline__ double divide_by(double x, double d, double r) {
   double q = x * r;
   q = fma(fma(-q, d, x), r, q);
