@@ -23,7 +23,9 @@
 // over the device (rank_update_kernel) in between.  Solves with few right-hand sides take one launch
 // per 64 rows and direction (trsv_block_kernel), others recurse on 64-row blocks and bzg_dgemm.
 // n = 3000 with 16 right-hand sides: 12.6 ms; 28.1 ms with leaves of 8 columns and dgetrf2's recursion
-// down to them (708 triangular solves of 32 rows, 796 small products).  n = 8192: 56 ms (98 ms).
+// down to them (708 triangular solves of 32 rows, 796 small products).  n = 8192: 55 ms (99 ms), 16384 349
+// (420), 25000 928 (1168): above 8192 rows a leaf holds two columns, above 16384 one, and those
+// instances spill (48 and 20 registers a lane).
 #include "common.hpp"
 
 #include <cfloat>

@@ -36,7 +36,7 @@ namespace {
 
 constexpr int NT = 64;        // threads per workgroup: one wavefront per system
 constexpr int NW = NT / 64;   // wavefronts per workgroup
-constexpr int NB = 16;        // panel width of lu_factor (FP32): NM / 64 rows x NB values per lane in registers
+constexpr int NB = 16;        // panel width of lu_factor32: NM / 64 rows x NB values per lane in registers
 constexpr int NMAX = 512;     // largest system order
 constexpr int NSMALL = 256;   // systems up to this order use the NM = 256 kernels
 constexpr int RMAX = 8;       // largest number of right-hand sides
@@ -44,10 +44,10 @@ constexpr int UPAD = 16;      // row padding of the U12 buffer (conflict-free MF
 
 // NM: the largest order a kernel instance handles (256 or 512); it sizes the LDS buffers and
 // the register panel (NM / 64 rows per lane).
-template <typename T, int NM>
-struct FactorShm {
-  T panel[NM][NB + 1];      // L11 / L21 of the current panel (rows beyond n are zero)
-  T ublk[NB][NM + UPAD];    // U12 of the current panel
+template <int NM>
+struct FactorShm32 {
+  float panel[NM][NB + 1];    // L11 / L21 of the current panel (rows beyond n are zero)
+  float ublk[NB][NM + UPAD];  // U12 of the current panel
 };
 
 template <typename T, int NM>
@@ -70,20 +70,6 @@ struct Misc {
   int flag;
 };
 
-template <typename T>
-struct MfmaLU;
-template <>
-struct MfmaLU<float> {
-  using acc_t = f4;
-  __device__ static acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static int row(int i, int lane) { return 4 * (lane / 16) + i; }
-};
-
-template <typename T>
-__device__ __forceinline__ T tabs(T v) { return v < T(0) ? -v : v; }
-
 // Value of lane `src` (wave-uniform) broadcast to the wavefront.
 __device__ __forceinline__ double bcast(double v, int src) {
   const long long b = __double_as_longlong(v);
@@ -95,14 +81,13 @@ __device__ __forceinline__ float bcast(float v, int src) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
 }
 
+// ---- FP32 factorisation (mixed solver, orders 257..512) ------------------------------------------
 // LU factorisation of the n x n row-major matrix A (leading dimension lda) in place.
 // Writes 1-based pivots to ipiv (may be null) and the row permutation to misc.perm.
 // Returns info (0 or 1-based index of the first exactly-zero pivot).
-template <typename T, int NM>
-__device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int32_t* __restrict__ ipiv,
-                         FactorShm<T, NM>& sh, Misc<NM>& misc) {
-  using MF = MfmaLU<T>;
-  using acc_t = typename MF::acc_t;
+template <int NM>
+__device__ __forceinline__ int lu_factor32(float* __restrict__ A, int n, int lda, int32_t* __restrict__ ipiv,
+                                           FactorShm32<NM>& sh, Misc<NM>& misc) {
   constexpr int Q = NM / 64;  // panel rows per lane
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int info = 0;
@@ -121,7 +106,7 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
     // butterfly over the wavefront and v_readlane broadcasts of the pivot row: no LDS traffic
     // and no barrier per column.
     if (wave == 0) {
-      T P[Q][NB];
+      float P[Q][NB];
       int lpos[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
@@ -129,7 +114,7 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
         lpos[q] = (rr < m) ? rr : (1 << 20);  // rows beyond the matrix never become candidates
 #pragma unroll
         for (int c = 0; c < NB; ++c)
-          P[q][c] = (rr < m && c < nbe) ? A[(long)(j0 + rr) * lda + j0 + c] : T(0);
+          P[q][c] = (rr < m && c < nbe) ? A[(long)(j0 + rr) * lda + j0 + c] : 0.f;
       }
 #pragma unroll
       for (int jj = 0; jj < NB; ++jj) {
@@ -137,42 +122,23 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
           // Candidates: logical rows jj..m-1.  A NaN entry ranks below every number (as in
           // idamax, where NaN never compares greater) but above the non-candidates, so the
           // pivot is always a row of the matrix.  Ties: the lower logical row.
-          int p;
-          if constexpr (sizeof(T) == 4) {
-            // one 64-bit key per candidate: (|a| bits + 2, or 1 for NaN, 0 for a non-candidate)
-            // above (2^32 - 1 - logical row); the wavefront maximum is the pivot
-            unsigned long long key = 0ull;
+          // One 64-bit key per candidate: (|a| bits + 2, or 1 for NaN, 0 for a non-candidate)
+          // above (2^32 - 1 - logical row); the wavefront maximum is the pivot.
+          unsigned long long key = 0ull;
 #pragma unroll
-            for (int q = 0; q < Q; ++q) {
-              const bool cand = lpos[q] >= jj && lpos[q] < m;
-              const float a = (float)P[q][jj];
-              const unsigned hi = !cand ? 0u : (a != a ? 1u : (__float_as_uint(a) & 0x7FFFFFFFu) + 2u);
-              const unsigned long long k = ((unsigned long long)hi << 32) | (0xFFFFFFFFu - (unsigned)lpos[q]);
-              key = k > key ? k : key;
-            }
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) {
-              const unsigned long long o = __shfl_xor(key, off, 64);
-              key = o > key ? o : key;
-            }
-            p = (int)(0xFFFFFFFFu - (unsigned)__builtin_amdgcn_readfirstlane((int)(key & 0xFFFFFFFFull)));
-          } else {
-            double v = -1.0;
-            int r = 1 << 30;
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-              double a = (lpos[q] >= jj && lpos[q] < m) ? (double)tabs(P[q][jj]) : -1.0;
-              if (a != a) a = -0.5;
-              if (a > v || (a == v && lpos[q] < r)) { v = a; r = lpos[q]; }
-            }
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) {
-              const double ov = __shfl_xor(v, off, 64);
-              const int orr = __shfl_xor(r, off, 64);
-              if (ov > v || (ov == v && orr < r)) { v = ov; r = orr; }
-            }
-            p = __builtin_amdgcn_readfirstlane(r);
+          for (int q = 0; q < Q; ++q) {
+            const bool cand = lpos[q] >= jj && lpos[q] < m;
+            const float a = P[q][jj];
+            const unsigned hi = !cand ? 0u : (a != a ? 1u : (__float_as_uint(a) & 0x7FFFFFFFu) + 2u);
+            const unsigned long long k = ((unsigned long long)hi << 32) | (0xFFFFFFFFu - (unsigned)lpos[q]);
+            key = k > key ? k : key;
           }
+#pragma unroll
+          for (int off = 32; off >= 1; off >>= 1) {
+            const unsigned long long o = __shfl_xor(key, off, 64);
+            key = o > key ? o : key;
+          }
+          const int p = (int)(0xFFFFFFFFu - (unsigned)__builtin_amdgcn_readfirstlane((int)(key & 0xFFFFFFFFull)));
           // physical place of logical row p: the lane holding it (ballot) and its register row
           bool mine = false;
           int myq = 0;
@@ -183,16 +149,16 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
           const int pl = __builtin_amdgcn_readfirstlane(__ffsll((long long)hold) - 1);
           const int pq = __builtin_amdgcn_readlane(myq, pl);
           // pivot row values (physical row (pl, pq)), kept in scalar registers
-          T pr[NB];
+          float pr[NB];
 #pragma unroll
           for (int c = 0; c < NB; ++c) {
-            T cand = P[0][c];
+            float cand = P[0][c];
 #pragma unroll
             for (int q = 1; q < Q; ++q) cand = (pq == q) ? P[q][c] : cand;
             pr[c] = bcast(cand, pl);
           }
-          const T piv = pr[jj];
-          if (piv != T(0)) {
+          const float piv = pr[jj];
+          if (piv != 0.f) {
             if (lane == 0) {
               misc.piv[jj] = j0 + p;
               const int t = misc.perm[j0 + jj];
@@ -203,11 +169,11 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
 #pragma unroll
             for (int q = 0; q < Q; ++q)
               lpos[q] = (lpos[q] == jj) ? p : ((lpos[q] == p) ? jj : lpos[q]);
-            const T rinv = T(1) / piv;
+            const float rinv = 1.f / piv;
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
               if (lpos[q] > jj && lpos[q] < m) {
-                const T l = P[q][jj] * rinv;
+                const float l = P[q][jj] * rinv;
                 P[q][jj] = l;
                 // constant trip count (c > jj folds after the jj loop is unrolled): a loop
                 // starting at jj + 1 would be unrolled first with a run-time trip count and
@@ -236,7 +202,7 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
             if (c < nbe) A[(long)(j0 + lr) * lda + j0 + c] = P[q][c];
             sh.panel[lr][c] = P[q][c];
           } else {
-            sh.panel[rr][c] = T(0);
+            sh.panel[rr][c] = 0.f;
           }
         }
       }
@@ -270,12 +236,12 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
     const int other = n - nbe;
     for (int oc = tid; oc < other; oc += NT) {
       const int c = oc < j0 ? oc : oc + nbe;
-      T top[NB], low[NB];
+      float top[NB], low[NB];
 #pragma unroll
       for (int jj = 0; jj < NB; ++jj) {
         const int st = misc.swsrc[jj], sl = misc.swsrc[NB + jj];
-        top[jj] = (st >= 0) ? A[(long)st * lda + c] : T(0);
-        low[jj] = (sl >= 0) ? A[(long)sl * lda + c] : T(0);
+        top[jj] = (st >= 0) ? A[(long)st * lda + c] : 0.f;
+        low[jj] = (sl >= 0) ? A[(long)sl * lda + c] : 0.f;
       }
       if (c > j0) {  // right of the panel: U12 column
 #pragma unroll
@@ -299,7 +265,7 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
       const int padded = (rem + 15) & ~15;
       for (int e = tid; e < NB * (padded - rem); e += NT) {
         const int rr = e / (padded - rem), cc = rem + e % (padded - rem);
-        sh.ublk[rr][cc] = T(0);
+        sh.ublk[rr][cc] = 0.f;
       }
     }
     __syncthreads();
@@ -308,20 +274,20 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
     // Each wavefront takes its tiles in batches of TB: all loads of a batch are issued before
     // the MFMAs, so a batch costs one HBM/L2 round trip instead of one per tile.
     if (rem > 0) {
-      constexpr int TB = (sizeof(T) == 8 ? 16 : 32) / (NM > 256 ? 2 : 1);  // register budget
+      constexpr int TB = NM > 256 ? 16 : 32;  // register budget
       const int tiles = (rem + 15) / 16;
       const int r0 = j0 + NB;
       const int total = tiles * tiles;
       for (int t0 = wave; t0 < total; t0 += NW * TB) {
-        acc_t acc[TB];
+        f4 acc[TB];
 #pragma unroll
         for (int q = 0; q < TB; ++q) {
           const int t = t0 + NW * q;
           const int ti = t / tiles, tj = t % tiles;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int gr = r0 + ti * 16 + MF::row(i, lane), gc = r0 + tj * 16 + lane % 16;
-            acc[q][i] = (t < total && gr < n && gc < n) ? A[(long)gr * lda + gc] : T(0);
+            const int gr = r0 + ti * 16 + 4 * (lane / 16) + i, gc = r0 + tj * 16 + lane % 16;
+            acc[q][i] = (t < total && gr < n && gc < n) ? A[(long)gr * lda + gc] : 0.f;
           }
         }
 #pragma unroll
@@ -331,9 +297,9 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
             const int ti = t / tiles, tj = t % tiles;
 #pragma unroll
             for (int kk = 0; kk < NB; kk += 4) {
-              const T a = -sh.panel[NB + ti * 16 + lane % 16][kk + lane / 16];
-              const T b = sh.ublk[kk + lane / 16][tj * 16 + lane % 16];
-              acc[q] = MF::mma(a, b, acc[q]);
+              const float a = -sh.panel[NB + ti * 16 + lane % 16][kk + lane / 16];
+              const float b = sh.ublk[kk + lane / 16][tj * 16 + lane % 16];
+              acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[q], 0, 0, 0);
             }
           }
         }
@@ -343,7 +309,7 @@ __device__ __forceinline__ int lu_factor(T* __restrict__ A, int n, int lda, int3
           const int ti = t / tiles, tj = t % tiles;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int gr = r0 + ti * 16 + MF::row(i, lane), gc = r0 + tj * 16 + lane % 16;
+            const int gr = r0 + ti * 16 + 4 * (lane / 16) + i, gc = r0 + tj * 16 + lane % 16;
             if (t < total && gr < n && gc < n) A[(long)gr * lda + gc] = acc[q][i];
           }
         }
@@ -367,7 +333,8 @@ struct Misc64 {
 // per 32 columns (orders up to 256).  Updated after every 8 columns it was four times that.  Beside
 // it, the wavefront waits: on memory between the phases and on the chain of a column step (2000 cycles).
 // So the orders up to 256 run two wavefronts a SIMD: 256 registers, LDS below 20 KB (U12 goes through
-// it 16 rows at a time, interchanged rows are gathered from memory and not staged in it).
+// it 16 rows at a time, interchanged rows are gathered from memory and not staged in it).  At 256 registers the
+// compiler spills 68 a lane (276 bytes of scratch), as it does in the solve alone (getrs_batched_kernel: 69).
 // 10,000 systems of orders 4..256, 1..8 right-hand sides, with their solves: 5.4 ms (11.5 ms with
 // panels of 8; 6.3 ms with one wavefront a SIMD).  With one, a wavefront's time was: tiles 19 %,
 // column steps 19 %, the solves 22 %, the second panel's update 9 %, U12 8 %, the rest loads and interchanges.
@@ -662,7 +629,7 @@ __device__ __forceinline__ void update_columns64(double* __restrict__ A, int n, 
   }
 }
 
-// LU factorisation of the n x n row-major matrix A (leading dimension lda) in place; as lu_factor.
+// LU factorisation of the n x n row-major matrix A (leading dimension lda) in place; as lu_factor32.
 template <int NM>
 __device__ __forceinline__ int lu_factor64(double* __restrict__ A, int n, int lda, int32_t* __restrict__ ipiv,
                                            FactorShm64<NM>& sh, Misc64<NM>& misc) {
@@ -839,18 +806,18 @@ __device__ __forceinline__ int next_system(int* counter, Shm& misc) {
   return s;
 }
 
-// ---- plain FP64 (or FP32) dgesv / dgetrf: A and B in place ------------------------------
+// ---- plain FP64 dgesv / dgetrf: A and B in place ---------------------------------------
 // MODE 0 (gesv): factor A, solve B.  MODE 1 (getrf): factor A only (rv may be null).
 // NM = NSMALL: takes the systems of order <= NSMALL from the (ordered) index range and skips
 // the others; NM = NMAX: takes the systems listed in big_list (orders NSMALL+1 .. NMAX).
 // Systems outside 1..NMAX / 0..RMAX were marked info = -1 by classify_kernel.
-template <typename T, int NM>
+template <int NM>
 __global__ __launch_bounds__(NT, NM == NSMALL ? 2 : 1) void gesv_batched_kernel(int count, const int32_t* __restrict__ nv,
                                                           const int32_t* __restrict__ rv,
                                                           const int64_t* __restrict__ a_off,
                                                           const int64_t* __restrict__ b_off,
                                                           const int64_t* __restrict__ p_off,
-                                                          T* __restrict__ A, T* __restrict__ B,
+                                                          double* __restrict__ A, double* __restrict__ B,
                                                           int32_t* __restrict__ ipiv,
                                                           int32_t* __restrict__ info,
                                                           const int32_t* __restrict__ order,
@@ -870,17 +837,17 @@ __global__ __launch_bounds__(NT, NM == NSMALL ? 2 : 1) void gesv_batched_kernel(
     const int s = (NM != NSMALL) ? big_list[idx] : (order ? order[idx] : idx);
     const int n = nv[s], nrhs = rv ? rv[s] : 0;
     if (NM == NSMALL && (n < 1 || n > NSMALL || nrhs < 0 || nrhs > RMAX)) continue;
-    T* a = A + a_off[s];
-    T* b = (mode != 1) ? B + b_off[s] : nullptr;
+    double* a = A + a_off[s];
+    double* b = (mode != 1) ? B + b_off[s] : nullptr;
     const int inf = lu_factor64<NM>(a, n, n, ipiv ? ipiv + p_off[s] : nullptr, sh.f, misc);
     if (tid == 0 && info) info[s] = inf;
     if (inf == 0 && mode != 1) {
       for (int e = tid; e < n * RMAX; e += NT) {
         const int i = e / RMAX, c = e % RMAX;
-        sh.s.x[e] = (c < nrhs) ? b[(long)misc.perm[i] * nrhs + c] : T(0);
+        sh.s.x[e] = (c < nrhs) ? b[(long)misc.perm[i] * nrhs + c] : 0.0;
       }
       __syncthreads();
-      lu_solve<T>(a, n, n, sh.s.x, nrhs, sh.s.diag);
+      lu_solve<double>(a, n, n, sh.s.x, nrhs, sh.s.diag);
       for (int e = tid; e < n * nrhs; e += NT) b[e] = sh.s.x[(e / nrhs) * RMAX + e % nrhs];
     }
     __syncthreads();
@@ -962,7 +929,7 @@ __global__ __launch_bounds__(NT) void dsgesv_batched_kernel(
     int* counter, float* __restrict__ ws32, int32_t* __restrict__ fallback_list,
     int* fallback_count, double tol, int max_iter) {
   __shared__ union {
-    FactorShm<float, NM> f;
+    FactorShm32<NM> f;
     IRShm<NM> ir;
   } sh;
   __shared__ Misc<NM> misc;
@@ -1027,7 +994,7 @@ __global__ __launch_bounds__(NT) void dsgesv_batched_kernel(
     const double eps = tol > 0 ? tol : 0x1.0p-53;
     const double cte = anrm * eps * sqrt((double)n);
     __syncthreads();
-    const int inf32 = lu_factor<float, NM>(W, n, n, nullptr, sh.f, misc);
+    const int inf32 = lu_factor32<NM>(W, n, n, nullptr, sh.f, misc);
     int it_out = -2;
     if (inf32 == 0) {
       // x = FP32 solve of P b
@@ -1288,10 +1255,10 @@ bzg_status lu_batched_scratch(bzg_context* ctx, int mode, int64_t count, const i
       hipLaunchKernelGGL((getrs_batched_kernel<NSMALL, 2>), grid, dim3(NT), 0, ctx->stream, (int)count, n, nrhs, a_off,
                          b_off, p_off, A, B, ipiv, info, order, list, list_count, counters + 0);
   } else {
-    hipLaunchKernelGGL((gesv_batched_kernel<double, NMAX>), grid_big, dim3(NT), 0, ctx->stream, (int)count, n, nrhs,
+    hipLaunchKernelGGL(gesv_batched_kernel<NMAX>, grid_big, dim3(NT), 0, ctx->stream, (int)count, n, nrhs,
                        a_off, b_off, p_off, A, B, ipiv, info, order, list, list_count, counters + 2, mode);
     BZG_LAUNCH_CHECK();
-    hipLaunchKernelGGL((gesv_batched_kernel<double, NSMALL>), grid, dim3(NT), 0, ctx->stream, (int)count, n, nrhs, a_off,
+    hipLaunchKernelGGL(gesv_batched_kernel<NSMALL>, grid, dim3(NT), 0, ctx->stream, (int)count, n, nrhs, a_off,
                        b_off, p_off, A, B, ipiv, info, order, list, list_count, counters + 0, mode);
   }
   BZG_LAUNCH_CHECK();
