@@ -626,8 +626,7 @@ bzg_status launch_shape(bzg_context* ctx, int shape, int64_t m, int64_t n, int64
 constexpr int64_t kMaxK = INT32_MAX - 127;
 
 // Tile choice by size only (never by load), so a product's result never depends on what
-// else is running: the tuned shape of the size class if there is one, else a heuristic
-// (large tiles cut L2->LDS traffic; small tiles keep >= ~256 workgroups in flight).
+// else is running: the tuned shape of the size class if there is one, else heuristic_shape's.
 template <typename T>
 bzg_status gemm_dispatch(bzg_context* ctx, int64_t m, int64_t n, int64_t k, T alpha, const T* A,
                          int64_t lda, const T* B, int64_t ldb, T beta, T* C, int64_t ldc, bool ta = false,

@@ -358,7 +358,7 @@ bzg_status launch_solves(bzg_server* s, Group* g) {
 
 // A solve of order 257..512 on its own: the batched mixed solver's kernel for these orders
 // takes one wavefront per system (about 10 ms for n = 512), the single-system FP64 LU
-// (bzg_dgetrf + bzg_dgetrs: recursive, MFMA trailing updates) a few ms.  The result is FP64
+// (bzg_dgetrf + bzg_dgetrs: panels of 64 columns, MFMA trailing updates) a few ms.  The result is FP64
 // LU's (iterations = -1, as for a fallback); info comes back with the group's event.
 bzg_status launch_direct(bzg_server* s, Group* g) {
   bzg_context* c = s->ctx[g->stream];
