@@ -565,22 +565,22 @@ TuneKey tune_key(int type, int64_t m, int64_t n, int64_t k) {
 }
 
 // Shapes: 0 = 32x32, 1 = 64x64, 2 = 128x128 tiles; 3 = 128x256 (64x128 per wavefront, FP32
-// only: its accumulators need 128 registers, 256 in FP64) -- 123.8 against 116.1 TFLOP/s at
-// 8192^3, 112.0 against 102.7 at 4096^3.
+// only: its accumulators need 128 registers, 256 in FP64).  131 TFLOP/s at 8192^3 and 4096^3; 128x128, once
+// behind, is at 136 and 133 now, which the rule does not use yet.
 template <typename T>
 constexpr int kShapes = sizeof(T) == 4 ? 4 : 3;
 constexpr int kShortK = 4;  // FP32 only, by rule: 64x64 with slabs of 16 and one ahead, as in the grouped kernel
 
-// Tiles against the 256 CUs, from products of 64 .. 4096 rows and columns with k = 64, 300, 1500 (us,
+// Tiles against the 256 CUs, from products of 64 .. 8192 rows and columns with k = 20 .. 8192 (us,
 // FP64 / FP32).  A large tile reads less per flop but leaves CUs idle in its last round: 128 x 128
-// only from 960 tiles and with 92 % of the rounds' slots filled (4096^2, k = 4096: 2015 FP64 against
-// 2070 with 64 x 64; k = 1500, 3700^2, 841 tiles: 802 / 420 against 693 / 379; 2936^2, 529 tiles: 632 /
-// 326 against 457 / 253); FP32's 128 x 256 likewise from 480 tiles.  64 x 64 from 600 tiles (2000^2, k =
-// 1500: 249 / 137 against 291 / 171 with 32 x 32; 1500^2, 576 tiles: 190 / 103 against 169 / 103), and
-// from 200 for short k, where the loads ahead of the first product are most of the time (1000^2,
-// k = 64: 8.2 / 6.8 against 9.0 / 7.4).  FP32 up to k = 64 with shallow slabs, which leave less of the last one
-// outside K (1500^2, k = 20: 6.3 us, 8.8 with slabs of 32, both operands transposed 6.5, 9.1; 2000^2, k = 48:
-// 9.6, 10.8; 1200^2, k = 64: 7.0, 7.5); from k = 100 the deep ones are ahead (1000^2: 7.3).
+// only from 960 tiles and with 92 % of the rounds' slots filled (8192^3: 16.1 ms / 8.1 against 16.9 / 8.5 with
+// 64 x 64; 4096^3: 2025 / 1031 against 1993 / 1077; k = 1500, 3700^2, 841 tiles: 749 / 384 against 644 / 356;
+// 2936^2, 529 tiles: 615 / 293 against 419 / 232); FP32's 128 x 256 likewise from 480 tiles.  64 x 64 from 600
+// tiles (2000^2, k = 1500: 193 / 108 against 248 / 146 with 32 x 32; 1500^2, 576 tiles: 143 / 83 against 141 /
+// 83), and from 200 for short k, where the loads ahead of the first product are most of the time (1000^2,
+// k = 64: 7.0 / 5.6 against 7.8 / 6.3).  FP32 below k = 64 with shallow slabs, which leave less of the last
+// one outside K (1500^2, k = 20: 6.4 us, 8.7 with slabs of 32; 2000^2, k = 48: 9.8, 10.7); at 64 the deep ones
+// are ahead (1200^2: 6.6, 6.9).
 template <typename T>
 int heuristic_shape(int64_t m, int64_t n, int64_t k) {
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
@@ -588,7 +588,7 @@ int heuristic_shape(int64_t m, int64_t n, int64_t k) {
   const int64_t t256 = tiles(128, 256), t128 = tiles(128, 128), t64 = tiles(64, 64);
   if (sizeof(T) == 4 && t256 >= 480 && filled(t256)) return 3;
   if (t128 >= 960 && filled(t128)) return 2;
-  if (sizeof(T) == 4 && t64 >= 200 && k <= 64) return kShortK;
+  if (sizeof(T) == 4 && t64 >= 200 && k < 64) return kShortK;
   if (t64 >= 600 || (t64 >= 200 && k <= (sizeof(T) == 8 ? 128 : 512))) return 1;
   return 0;
 }
